@@ -148,6 +148,38 @@ def test_gemm_every_plan(gpu, wtype, plan):
         gpu.tune("gemm_plan", "")
 
 
+# The k-wavefront kernel's tiles (pipeline 3), over rows and columns that end inside a tile, k steps that
+# leave wavefronts with none (64, 320) or unequal shares (960), a row count that needs padding columns
+# (257 -> 320) and dual columns.
+@pytest.mark.parametrize("wtype", [wa.Q8_0, wa.Q4_0, wa.F16])
+@pytest.mark.parametrize("plan", ["32,32,1,1,2,1,3,8", "32,64,1,1,2,1,3,8", "64,64,1,1,2,1,3,4"])
+def test_gemm_k_wavefronts(gpu, wtype, plan):
+    gpu.tune("gemm_plan", plan)
+    try:
+        for m, n, k, d in ((1, 64, 64, 0), (33, 257, 320, 0), (95, 320, 960, 64), (64, 128, 2048, 0)):
+            w = np.random.default_rng(k).normal(0, 0.02, (n, k)).astype(np.float32)
+            raw, bias = ox.quantize(w, wtype), rnd(n + d, 2)
+            l = gpu.linear([(raw, wtype, k, n)], bias)
+            ol = ox.Linear(wtype, k, [(raw, n)], bias[:n])
+            a = rnd(m * k, 3).reshape(m, k)
+            c0 = rnd(m * l.width, 4).reshape(m, l.width)
+            ab = gpu.upload(a)
+            ah = gpu.upload(a.astype(np.float16))
+            for e, alpha in ((wa.BIAS, 0.0), (wa.RESIDUAL, 0.5), (wa.SILU, 0.0)):
+                cb = gpu.upload(c0)
+                gpu.gemm(ab, l, cb, m, e, alpha)
+                want = ox.gemm_wide(a, ol, m, e, alpha, c=c0, bias2=bias[n:] if d else None, dual=d)
+                tol = 2e-5 * max(1.0, float(np.abs(want).max()))  # f32 sums in another order, as above
+                close(gpu.read(cb, c0.shape), want, tol=tol, what=f"plan {plan} type {wtype} {m}x{n}x{k} epi {e}")
+                if e == wa.SILU:  # f16 outputs: the f32 ones rounded once (2^-11 relative)
+                    hb = gpu.buffer((c0.size + 1) // 2)
+                    gpu.gemm_h(ah, l, hb, m, e, 0.0, out16=True)
+                    got = gpu.read(hb, c0.shape, np.float16).astype(np.float32)
+                    close(got, want, tol=tol + 2.0 ** -11 * float(np.abs(want).max()), what=f"plan {plan} f16 {m}x{n}x{k}")
+    finally:
+        gpu.tune("gemm_plan", "")
+
+
 @pytest.mark.parametrize("plan", ["96,128,1,4,3,1,0,2", "96,64,1,2,2,4", "64,64,2,2,3,1"])
 def test_gemm_tile_orders_agree(gpu, plan):
     # The order in which XCDs take the tiles (groups of 1, 2, 3 and all row tiles, column by column

@@ -18,6 +18,9 @@
 // few output tiles for the 256 CUs split k 2 or 4 ways into f32 partial sums that a second kernel
 // adds in a fixed order before the epilogue.
 //
+// Few tiles (gemm_kw_kernel): the wavefronts of a workgroup split k and read W from tiles laid out for
+// their loads when the weights are created (weight_tiles_kernel).
+//
 // Fallback kernel (gemm_reg_kernel; any k % 32 == 0 and F32 weights): a double-buffered a tile in
 // LDS and W blocks loaded straight into registers.
 #include <algorithm>
@@ -97,12 +100,34 @@ GemmPlan gemm_plan_for(const wh_ctx *ctx, int m, int cols, int k) {
     // tiles of one row of 2 wavefronts in two k groups, one workgroup per CU (11.7 against 12.7 µs
     // in the step for 64×64 tiles; 12.2 with 4 slots).
     p = {96, 64, 1, 2, 2, 1, 0, 2};
+  // Few tiles: wavefronts that split k (gemm_kw_kernel), the smallest of its tiles that still run at once
+  // (one workgroup per CU), whose chain of steps is then the shortest.  Both sides inside the encoder
+  // call, µs per call with that one layer on either kernel: 60 Parakeet frames (32×32 tiles, 32×64 for the
+  // wider ones) 2 289 against 2 073 for the 1024 × 1024 projections, 2 298 for 4096 × 1024, all of them
+  // 2 807; 31 GigaAM frames 1 915 against 1 380 all together.  64×64 tiles up to two per CU where 96-row
+  // tiles would not run at once either (500 frames, 4096 × 1024: 3 244 against 3 132), but not past 1024
+  // rows (Whisper's 1500 × 1280 × 1280: 723 against 708 per four layers), and not over a long k, which
+  // the split plans above walk faster (500 frames' 1024 × 4096: 3 400 on 64×64 tiles here, 3 319 split,
+  // 3 132 on 32×64; 750 frames': 4 071 against 3 944).
+  {
+    const long t32 = (long)((cols + 31) / 32) * ((m + 31) / 32), t3264 = (long)((cols + 63) / 64) * ((m + 31) / 32);
+    const long t96 = (long)((cols + 63) / 64) * ((m + 95) / 96);
+    if ((size_t)m * k < ((size_t)1 << 30)) {  // 32-bit byte offsets into a
+      if (t32 <= cus) p = {32, 32, 1, 1, 2, 1, PIPE_KW, 8};
+      else if (t3264 <= cus) p = {32, 64, 1, 1, 2, 1, PIPE_KW, 8};
+      else if (k <= 2048 && (t64 <= cus || (m < 1024 && t64 <= 2L * cus && t96 > cus))) p = {64, 64, 1, 1, 2, 1, PIPE_KW, 4};
+    }
+  }
   if (ctx->gemm_plan[0]) {  // tuning override (wh_tune "gemm_plan"): bm, bn, wm, wn, stages, split, pipeline, kgroups
     const int *o = ctx->gemm_plan;
     p = {o[0], o[1], o[2], o[3], o[4], o[5], o[6], std::max(1, o[7])};
   }
   for (const auto &o : ctx->gemm_shape_plans)  // tuning override for one shape (wh_tune "gemm_shape_plans")
     if (o[0] == m && o[1] == cols && o[2] == k) p = {o[3], o[4], o[5], o[6], o[7], o[8], o[9], std::max(1, o[10])};
+  if (p.pipe == PIPE_KW) {  // (any k steps: a wavefront may have one less than another, or none)
+    p.split = 1;
+    return p;
+  }
   // Whole k steps per split and k group.
   if (k % (64 * p.wk)) p.wk = 1;
   if (k % (64 * p.wk * p.split)) p.split = 1;
@@ -126,6 +151,50 @@ bool lds_path(const wh_linear *l, const void *c, int ldc) {
          ldc % 8 == 0 && (uintptr_t)c % 16 == 0;
 }
 
+
+// The k-wavefront kernel's weight tiles from the GGUF bytes (see WTile): a lane of a tile per thread.
+template <int WT>
+__global__ __launch_bounds__(256) void weight_tiles_kernel(const uint8_t *__restrict__ w, uint8_t *__restrict__ wt, int rows,
+                                                           int nkt, size_t row_bytes, size_t lanes) {
+  constexpr int BLK = WT == WH_Q8_0 ? 34 : 18;
+  for (size_t e = (size_t)blockIdx.x * 256 + threadIdx.x; e < lanes; e += (size_t)gridDim.x * 256) {
+    const size_t tile = e / 64;
+    const int lane = e % 64, g = lane / 32, row = (int)(tile / nkt) * 32 + lane % 32, kt = (int)(tile % nkt);
+    uint8_t *dst = wt + tile * WTile<WT>::BYTES;
+    const uint8_t *src = w + (size_t)row * row_bytes;
+    u32x4 q[WTile<WT>::LOADS] = {};
+    uint32_t sc = 0;
+    if (row < rows) {
+      if constexpr (WT == WH_F16) {
+        // (rows of k % 64 == 0 halves: 16-byte aligned)
+#pragma unroll
+        for (int s = 0; s < 4; s++) q[s] = *(const u32x4 *)(src + 128 * (size_t)kt + 32 * s + 16 * g);
+      } else {
+        const uint16_t *b = (const uint16_t *)(src + (size_t)kt * 2 * BLK);  // the step's block pair
+        sc = b[0] | (uint32_t)b[BLK / 2] << 16;
+        if constexpr (WT == WH_Q8_0) {
+#pragma unroll
+          for (int s = 0; s < 4; s++) {  // substep s: bytes 16·(s % 2) + 8g .. of block s / 2
+            const uint16_t *d = b + (s / 2) * (BLK / 2) + 1 + 8 * (s & 1) + 4 * g;
+            q[s / 2][2 * (s & 1)] = d[0] | (uint32_t)d[1] << 16, q[s / 2][2 * (s & 1) + 1] = d[2] | (uint32_t)d[3] << 16;
+          }
+        } else {
+#pragma unroll
+          for (int s = 0; s < 4; s++) {  // element 16·(s % 2) + 8g + i of block s / 2: a nibble of byte 8g + i
+            const uint8_t *d = (const uint8_t *)b + (s / 2) * BLK + 2 + 8 * g;
+            uint32_t x = 0;
+#pragma unroll
+            for (int i = 0; i < 8; i++) x |= (uint32_t)(s & 1 ? d[i] >> 4 : d[i] & 15) << (4 * (i / 2) + 16 * (i & 1));
+            q[0][s] = x;
+          }
+        }
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < WTile<WT>::LOADS; i++) *(u32x4 *)(dst + 1024 * i + 16 * lane) = q[i];
+    if (WT != WH_F16 && g == 0) *(uint32_t *)(dst + WTile<WT>::DATA + 4 * lane) = sc;
+  }
+}
 
 // Scratch bytes for the split-k partial sums of an m-row GEMM (0 when it does not split).
 size_t split_bytes(const wh_ctx *ctx, const wh_linear *l, int m) {
@@ -189,6 +258,30 @@ int launch_typed(wh_ctx *ctx, const void *a, const wh_linear *l, void *c, int m,
 }
 
 }  // namespace
+
+size_t weight_tile_bytes(int type, int rows, int k) {
+  if (k % 64) return 0;
+  const size_t tiles = (size_t)((rows + 31) / 32) * (k / 64);
+  switch (type) {
+    case WH_Q8_0: return tiles * WTile<WH_Q8_0>::BYTES;
+    case WH_Q4_0: return tiles * WTile<WH_Q4_0>::BYTES;
+    case WH_F16: return tiles * WTile<WH_F16>::BYTES;
+  }
+  return 0;
+}
+
+int launch_weight_tiles(wh_ctx *ctx, const wh_linear *l) {
+  const size_t lanes = (size_t)((l->rows + 31) / 32) * (l->k / 64) * 64;
+  const int blocks = (int)std::min<size_t>((lanes + 255) / 256, 16384);
+  auto go = [&](auto kernel) { wh_launch(ctx, kernel, blocks, 256, 0, (const uint8_t *)l->w, l->wt, l->rows, l->k / 64, l->row_bytes, lanes); };
+  switch (l->type) {
+    case WH_Q8_0: go(weight_tiles_kernel<WH_Q8_0>); break;
+    case WH_Q4_0: go(weight_tiles_kernel<WH_Q4_0>); break;
+    case WH_F16: go(weight_tiles_kernel<WH_F16>); break;
+    default: return WH_OK;
+  }
+  return wh_launched(ctx, "weight tiles");
+}
 
 bool gemm_glu_ok(const wh_linear *l, const void *c) {
   return l && !l->dual && l->rows == l->cols && l->cols % 16 == 0 && lds_path(l, c, l->cols / 2);

@@ -17,6 +17,9 @@ struct GemmPlan {
   int bm, bn, wm, wn, ns, split, pipe = 0, wk = 1;
 };
 
+// GemmPlan::pipe of the k-wavefront kernel (gemm_kw_kernel): bm × bn tiles of wk wavefronts.
+constexpr int PIPE_KW = 3;
+
 // The launch plan of an m × cols × k GEMM (gemm.hip).
 GemmPlan gemm_plan_for(const wh_ctx *ctx, int m, int cols, int k);
 
@@ -446,23 +449,38 @@ __device__ __forceinline__ int epi_half(int r) {
 // rows give); a split GEMM stores its plain partial sums into plane tz instead.  A pass holds, for
 // every row group of RPW tile rows (one per row of wavefronts), PGR of its rows from row 32·i0: LDS
 // row r is tile row (r / PGR)·RPW + 32·i0 + r % PGR (PGR = RPW, i0 = 0: the whole tile in order).
-template <int NR, int RPW, int PGR, int BN, int NT, bool SPLIT, bool OUT16, bool TWO = false>
+template <int NR, int RPW, int PGR, int BN, int NT, bool SPLIT, bool OUT16, bool TWO = false, int NP = 1>
 __device__ __forceinline__ void store_c_tile(const LdsArgs &P, const float *cl, int crow, int tid, int m0, int n0,
                                              int tz, int i0, const float (&bb)[8], const float (&bd)[8],
-                                             const float *cl2 = nullptr, int ccol = 0) {
+                                             const float *cl2 = nullptr, int ccol = 0, int cpl = 0) {
   constexpr int G8 = BN / 8;
-  // The tile's sums: with TWO the two k groups' planes added as they are read (group 0's + group 1's).
+  // Rounds of NT 8-column items; where the items are no whole rounds, the threads past them are idle.
+  constexpr int ITEMS = NR * G8, ITS = (ITEMS + NT - 1) / NT;
+  constexpr bool PART = ITEMS % NT != 0;
+  // The tile's sums: with TWO the two k groups' planes added as they are read (group 0's + group 1's), with
+  // NP > 1 the NP planes of cpl floats, in order.
   auto rd4 = [&](int off) {
     float4 a = *(const float4 *)(cl + off);
     if constexpr (TWO) {
       const float4 b = *(const float4 *)(cl2 + off);
       a.x += b.x, a.y += b.y, a.z += b.z, a.w += b.w;
     }
+    if constexpr (NP > 1) {
+#pragma unroll
+      for (int p = 1; p < NP; p++) {
+        const float4 b = *(const float4 *)(cl + p * cpl + off);
+        a.x += b.x, a.y += b.y, a.z += b.z, a.w += b.w;
+      }
+    }
     return a;
   };
   auto rd1 = [&](int off) {
     float a = cl[off];
     if constexpr (TWO) a += cl2[off];
+    if constexpr (NP > 1) {
+#pragma unroll
+      for (int p = 1; p < NP; p++) a += cl[p * cpl + off];
+    }
     return a;
   };
   // Row r's 8 columns from c8, in the read order of epi_half (x in column order).
@@ -474,7 +492,6 @@ __device__ __forceinline__ void store_c_tile(const LdsArgs &P, const float *cl, 
   };
   const int et = epi_lane<BN>(tid);  // the lane's place in the row-major rounds below
   const int m = P.m, rows = P.rows;
-  static_assert((NR * G8) % NT == 0, "whole rounds of column groups");
   static_assert(PGR % 32 == 0 && RPW % PGR == 0, "passes of whole 32-row groups");
   const int m0p = m0 + 32 * i0;  // tile row of LDS row r: m0p + trow(r)
   auto trow = [](int r) { return (r / PGR) * RPW + r % PGR; };
@@ -493,7 +510,6 @@ __device__ __forceinline__ void store_c_tile(const LdsArgs &P, const float *cl, 
         // blocked, along the columns in pairs of 8-row halves (a block's columns follow each other).
         // Every item's bias loaded before the first store (a load after a store to memory that may
         // alias it would wait for a round trip per item).
-        constexpr int ITS = (BM * G8 + NT - 1) / NT;
         float bi[ITS];
 #pragma unroll
         for (int it = 0; it < ITS; it++) {
@@ -524,8 +540,10 @@ __device__ __forceinline__ void store_c_tile(const LdsArgs &P, const float *cl, 
         static_assert(NT % BN == 0, "a fixed column per lane");
         const float b = n0 + tid % BN < P.cols ? P.bias[n0 + tid % BN] : 0.0f;
 #pragma unroll
-        for (int it = 0; it < BM * G8 / NT; it++) {
+        for (int it = 0; it < ITS; it++) {
           const int e = tid + it * NT, c = e % BN, r0 = 8 * (e / BN), row0 = m0p + trow(r0), col = n0 + c;
+          if constexpr (PART)
+            if (e >= ITEMS) continue;
           if (row0 >= h.rs || col >= P.cols) continue;
           half8 y;
 #pragma unroll
@@ -538,8 +556,10 @@ __device__ __forceinline__ void store_c_tile(const LdsArgs &P, const float *cl, 
         }
       } else {
 #pragma unroll
-        for (int it = 0; it < BM * G8 / NT; it++) {
+        for (int it = 0; it < ITS; it++) {
           const int e = et + it * NT, r = e / G8, c8 = 8 * (e % G8), row = m0p + trow(r), col = n0 + c8;
+          if constexpr (PART)
+            if (e >= ITEMS) continue;
           if (row + h.r0 >= h.rs || col >= P.cols) continue;
           half8 y;
           if (row < m) {
@@ -565,8 +585,10 @@ __device__ __forceinline__ void store_c_tile(const LdsArgs &P, const float *cl, 
       auto run = [&](auto E_c) {
         constexpr int E = decltype(E_c)::value;
 #pragma unroll
-        for (int it = 0; it < BM * G8 / NT; it++) {
+        for (int it = 0; it < ITS; it++) {
           const int e = et + it * NT, r = e / G8, c8 = 8 * (e % G8), row = m0p + trow(r), col = n0 + c8;
+          if constexpr (PART)
+            if (e >= ITEMS) continue;
           if (row >= m) continue;
           float x[8];
           rd8(r, c8, x);
@@ -624,8 +646,10 @@ __device__ __forceinline__ void store_c_tile(const LdsArgs &P, const float *cl, 
     }
   }
 #pragma unroll
-  for (int it = 0; it < BM * G8 / NT; it++) {
+  for (int it = 0; it < ITS; it++) {
     const int e = et + it * NT, r = e / G8, c8 = 8 * (e % G8), row = m0p + trow(r), col = n0 + c8;
+    if constexpr (PART)
+      if (e >= ITEMS) continue;
     if (row >= m || col >= P.cols) continue;  // cols % 32 == 0: a group is inside or past
     float x[8];
     rd8(r, c8, x);
@@ -1127,6 +1151,230 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void gemm_lds_kernel(LdsArgs P) 
   static_for<0, TM, PG>(pass);
 }
 
+// ------------------------------------------------------------------- wavefronts splitting k
+
+// W as the k-wavefront kernel reads it (wh_linear::wt, made from the GGUF bytes when the weights are
+// created): tiles of 32 rows × 64 k, [row tile][k step], rows past the last one zeros.  A tile holds the
+// MFMA operand bytes of lane l = 32g + r (row r, k half g) in the order the lanes load them, 16 bytes per
+// lane and load, so a load is 1 KiB of consecutive bytes:
+//   Q8_0  load i: block i's elements 8g .. 8g + 7, then 16 + 8g .. 16 + 8g + 7 (substeps 2i and 2i + 1);
+//   Q4_0  one load, dword s: substep s's 8 nibbles, element 2h at bits 4h, element 2h + 1 at bits 16 + 4h;
+//   F16   load s: substep s's 8 halves;
+// then, quantized, the two block scales of each row (f16 pairs).  The bytes are as many as in the file.
+template <int WT>
+struct WTile {
+  static constexpr int LOADS = WT == WH_Q8_0 ? 2 : WT == WH_Q4_0 ? 1 : 4;
+  static constexpr int DATA = 1024 * LOADS;
+  static constexpr int BYTES = DATA + (WT == WH_F16 ? 0 : 128);
+};
+
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+
+// The MFMA operand of substep S from a lane's loads of a tile: f16(q·d), as dequant_q8 / dequant_frag.
+template <int WT, int S>
+__device__ __forceinline__ half8 tile_frag(const u32x4 (&q)[WTile<WT>::LOADS], uint32_t sc) {
+  if constexpr (WT == WH_F16) {
+    return __builtin_bit_cast(half8, q[S]);
+  } else {
+    const half2 sv = __builtin_bit_cast(half2, sc);
+    const half2 d2 = {sv[S / 2], sv[S / 2]};
+    half2 p[4];
+    if constexpr (WT == WH_Q8_0) {
+      const uint32_t x0 = q[S / 2][2 * (S & 1)], x1 = q[S / 2][2 * (S & 1) + 1];
+      p[0] = i8_pair<false>(x0), p[1] = i8_pair<true>(x0), p[2] = i8_pair<false>(x1), p[3] = i8_pair<true>(x1);
+    } else {
+      const half2 bias = {(_Float16)1032.0f, (_Float16)1032.0f};  // 1024 + 8
+#pragma unroll
+      for (int h = 0; h < 4; h++)
+        p[h] = __builtin_bit_cast(half2, ((q[0][S] >> (4 * h)) & 0x000f000fu) | 0x64006400u) - bias;
+    }
+    half8 f;
+#pragma unroll
+    for (int h = 0; h < 4; h++) {
+      const half2 v = p[h] * d2;
+      f[2 * h] = v[0], f[2 * h + 1] = v[1];
+    }
+    return f;
+  }
+}
+
+struct KwArgs : LdsArgs {
+  const uint8_t *wt;  // W in tiles (WTile)
+};
+
+// c tile (32·TM) × (32·TN) per workgroup of WK wavefronts, each over its own 1/WK of the k steps (for
+// the whole tile): GEMMs of few tiles, whose time is the latency of a workgroup's chain of steps rather
+// than any throughput.  A wavefront shares nothing with the others until the end: it loads its a rows
+// and W tiles into registers two steps ahead, turns the a rows around in LDS of its own (two slots; a
+// wavefront's LDS operations run in order, so no barrier) and feeds the MFMAs, W straight from its
+// registers.  Splitting k over 4 or 8 wavefronts makes the chain 4 or 8 times shorter than in
+// gemm_lds_kernel, which walks the whole k with a barrier per step, and needs no partial sums in memory:
+// back to back with cold weights (~2.4 µs of each figure is the launch), 275×768×768 7.2 -> 4.5 µs,
+// 275×768×3072 13.8 (two splits and their finish) -> 7.6, 25×1024×1024 7.6 -> 4.3, 500×2048×1024
+// 10.1 -> 8.1.  The sums of the WK wavefronts are added in wavefront order through LDS planes.
+template <int WT, int TM, int TN, int WK, bool OUT16>
+__global__ __launch_bounds__(64 * WK) void gemm_kw_kernel(KwArgs P) {
+  constexpr int BM = 32 * TM, BN = 32 * TN, NT = 64 * WK, CROW = BN + 8, CPL = BM * CROW;
+  constexpr int A_ST = BM * 128;  // LDS bytes of one step's a rows
+  constexpr int RING = WK * 2 * A_ST, PLANES = WK * CPL * 4;
+  constexpr int NQ = WTile<WT>::LOADS, NA = 4 * TM;
+  __shared__ __attribute__((aligned(16))) uint8_t lds[RING > PLANES ? RING : PLANES];
+
+  if (P.skip && *P.skip == P.skip_val) return;  // c already holds this product
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  // The tile order of gemm_lds_kernel (contiguous runs of tiles per XCD, in groups of P.group row tiles).
+  int tx, ty;
+  {
+    const int nx = gridDim.x, ny = gridDim.y, total = nx * ny;
+    const int lin = blockIdx.x + nx * blockIdx.y, x = lin % 8, e = x * (total / 8) + min(x, total % 8) + lin / 8;
+    const int g0 = e / (P.group * nx) * P.group, gh = min(P.group, ny - g0), w = e - g0 * nx;
+    ty = g0 + w % gh;
+    tx = w / gh;
+  }
+  const int n0 = tx * BN, m0 = ty * BM, m = P.m, k = P.k;
+  const int lrow = lane & 31, g = lane >> 5;
+  const int nkt = k / 64, k0 = nkt * wave / WK, ns = nkt * (wave + 1) / WK - k0;  // this wavefront's steps
+
+  // Loads: 8 a rows of 128 bytes each (rows past m clamped: their products are discarded), W tiles
+  // (tiles past the last one likewise).
+  uint32_t aoff[NA];
+#pragma unroll
+  for (int i = 0; i < NA; i++) aoff[i] = (uint32_t)(((size_t)min(m0 + 8 * i + lane / 8, m - 1) * k + 8 * (lane % 8)) * 2);
+  const uint8_t *ab = (const uint8_t *)P.a + (size_t)k0 * 128;
+  const uint8_t *wb[TN];
+#pragma unroll
+  for (int j = 0; j < TN; j++)
+    wb[j] = P.wt + ((size_t)min(n0 / 32 + j, (P.rows + 31) / 32 - 1) * nkt + k0) * WTile<WT>::BYTES;
+  auto load_a = [&](u32x4 (&r)[NA], int t) {
+    const uint8_t *b = ab + (size_t)t * 128;
+#pragma unroll
+    for (int i = 0; i < NA; i++) r[i] = *(const u32x4 *)(b + aoff[i]);
+  };
+  auto load_w = [&](u32x4 (&q)[TN][NQ], uint32_t (&s)[TN], int t) {
+#pragma unroll
+    for (int j = 0; j < TN; j++) {
+      const uint8_t *b = wb[j] + (size_t)t * WTile<WT>::BYTES;
+#pragma unroll
+      for (int i = 0; i < NQ; i++) q[j][i] = *(const u32x4 *)(b + 1024 * i + 16 * lane);
+      s[j] = WT == WH_F16 ? 0u : *(const uint32_t *)(b + WTile<WT>::DATA + 4 * lrow);
+    }
+  };
+  // The a rows in LDS: 16-byte chunk c of row r at (c + r / 2) % 8, free of bank conflicts (gemm_lds_kernel).
+  uint8_t *mine = lds + wave * 2 * A_ST;
+  auto write_a = [&](const u32x4 (&r)[NA], int slot) {
+#pragma unroll
+    for (int i = 0; i < NA; i++)
+      *(u32x4 *)(mine + slot * A_ST + 1024 * i + 128 * (lane / 8) + 16 * ((lane % 8 + 4 * i + lane / 16) & 7)) = r[i];
+  };
+  uint32_t a_off[4];
+#pragma unroll
+  for (int s = 0; s < 4; s++) a_off[s] = 128 * lrow + 16 * ((2 * s + g + (lrow >> 1)) & 7);
+  auto read_a = [&](half8 (&f)[TM], int slot, int s) {
+#pragma unroll
+    for (int i = 0; i < TM; i++) f[i] = *(const half8 *)(mine + slot * A_ST + a_off[s] + 4096 * i);
+  };
+
+  constexpr int G8 = BN / 8;
+  static_assert(NT % G8 == 0 && NT % BN == 0, "fixed column group per thread");
+  floatx16 acc[TM][TN];
+#pragma unroll
+  for (int i = 0; i < TM; i++)
+#pragma unroll
+    for (int j = 0; j < TN; j++) acc[i][j] = floatx16{};
+  u32x4 ra[2][NA], wq[2][TN][NQ];
+  uint32_t ws[2][TN];
+  half8 af[2][TM];
+#pragma unroll
+  for (int p = 0; p < 2; p++)
+    if (p < ns) {
+      load_a(ra[p], p);
+      load_w(wq[p], ws[p], p);
+    }
+  // The bias of the thread's column group, needed after the loop.
+  const int ecol = n0 + 8 * (epi_lane<BN>(tid) % G8);
+  float bb[8] = {}, bd[8] = {};
+  if (ecol < P.cols) {
+    const float4 b0 = *(const float4 *)(P.bias + ecol), b1 = *(const float4 *)(P.bias + ecol + 4);
+    bb[0] = b0.x, bb[1] = b0.y, bb[2] = b0.z, bb[3] = b0.w, bb[4] = b1.x, bb[5] = b1.y, bb[6] = b1.z, bb[7] = b1.w;
+#pragma unroll
+    for (int q = 0; q < 8; q++)
+      if (ecol + q < P.dual) bd[q] = P.bias[P.cols + ecol + q];
+  }
+  if (ns > 0) {
+    write_a(ra[0], 0);
+    if (2 < ns) load_a(ra[0], 2);
+    read_a(af[0], 0, 0);
+  }
+  auto mma = [&](const half8 (&f)[TM], int set, auto s_c) {
+#pragma unroll
+    for (int j = 0; j < TN; j++) {
+      const half8 b = tile_frag<WT, decltype(s_c)::value>(wq[set][j], ws[set][j]);
+#pragma unroll
+      for (int i = 0; i < TM; i++) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(f[i], b, acc[i][j], 0, 0, 0);
+    }
+  };
+  // Step t, S = t % 2: its a rows are in slot S, step t + 1's in flight into ra[1 − S]; each substep's a
+  // fragments are read during the substep before it.  (Scheduling barriers between the substeps keep the
+  // loads where they are written: ahead of the MFMAs that hide them.)
+  auto step = [&](auto S_c, int t) {
+    constexpr int S = decltype(S_c)::value;
+    read_a(af[1], S, 1);
+    mma(af[0], S, std::integral_constant<int, 0>{});
+    __builtin_amdgcn_sched_barrier(0);
+    read_a(af[0], S, 2);
+    mma(af[1], S, std::integral_constant<int, 1>{});
+    __builtin_amdgcn_sched_barrier(0);
+    read_a(af[1], S, 3);
+    if (t + 1 < ns) {
+      write_a(ra[1 - S], 1 - S);
+      if (t + 3 < ns) load_a(ra[1 - S], t + 3);
+    }
+    mma(af[0], S, std::integral_constant<int, 2>{});
+    __builtin_amdgcn_sched_barrier(0);
+    if (t + 1 < ns) read_a(af[0], 1 - S, 0);
+    mma(af[1], S, std::integral_constant<int, 3>{});
+    if (t + 2 < ns) load_w(wq[S], ws[S], t + 2);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  for (int t0 = 0; t0 < ns; t0 += 2) unrolled_steps<0, 2>(step, t0, ns);
+
+  // Every wavefront's sums into a plane of its own (over the a rows: the barrier ends their reads), then
+  // the stores, which add the planes.  A tile of a transposed packed range column by column, as in
+  // gemm_lds_kernel.
+  constexpr int CCOL = BM + 4;
+  constexpr bool TCM = OUT16 && BN * CCOL <= CPL;
+  bool trt = false;
+  if constexpr (TCM) {
+#pragma unroll
+    for (int o = 0; o < 2; o++)
+      if (o < P.nho && P.ho[o].tr && n0 >= P.ho[o].col0 && n0 < P.ho[o].col0 + P.ho[o].cols) trt = true;
+  }
+  __syncthreads();
+  float *plane = (float *)lds + wave * CPL;
+  if (TCM && trt) {
+#pragma unroll
+    for (int i = 0; i < TM; i++)
+#pragma unroll
+      for (int j = 0; j < TN; j++)
+#pragma unroll
+        for (int v4 = 0; v4 < 4; v4++)
+          *(float4 *)(plane + (32 * j + lrow) * CCOL + 32 * i + 8 * v4 + 4 * g) =
+              make_float4(acc[i][j][4 * v4], acc[i][j][4 * v4 + 1], acc[i][j][4 * v4 + 2], acc[i][j][4 * v4 + 3]);
+  } else {
+#pragma unroll
+    for (int i = 0; i < TM; i++)
+#pragma unroll
+      for (int j = 0; j < TN; j++)
+#pragma unroll
+        for (int v = 0; v < 16; v++)
+          plane[(32 * i + 8 * (v >> 2) + 4 * g + (v & 3)) * CROW + 32 * j + lrow] = acc[i][j][v];
+  }
+  __syncthreads();
+  store_c_tile<BM, BM, BM, BN, NT, false, OUT16, false, WK>(P, (const float *)lds, CROW, tid, m0, n0, 0, 0, bb, bd, nullptr,
+                                                            TCM && trt ? CCOL : 0, CPL);
+}
+
 // Split-k finish: c = epi(Σ_z part[z] + bias) with the partial sums added in split order (the same
 // result on every run), dual outputs and padding columns as in the kernel above.
 template <bool OUT16>
@@ -1167,10 +1415,27 @@ int lds_launch(wh_ctx *ctx, dim3 grid, const LdsArgs &a, bool split, bool out16)
   }
 }
 
+// The k-wavefront kernel of plan p (*ok: built).
+template <int WT>
+int kw_launch(wh_ctx *ctx, dim3 grid, const KwArgs &a, const GemmPlan &p, bool out16, bool *ok) {
+#define KW(TM, TN, WK)                                                                              \
+  if (p.bm == 32 * TM && p.bn == 32 * TN && p.wk == WK && p.split == 1) {                           \
+    if (out16) wh_launch(ctx, gemm_kw_kernel<WT, TM, TN, WK, true>, grid, 64 * WK, 0, a);           \
+    else wh_launch(ctx, gemm_kw_kernel<WT, TM, TN, WK, false>, grid, 64 * WK, 0, a);                \
+    *ok = true;                                                                                     \
+  }
+  KW(1, 1, 8)
+  KW(1, 2, 8)
+  KW(2, 2, 4)
+#undef KW
+  return WH_OK;
+}
+
 template <int WT>
 int launch_lds_t(wh_ctx *ctx, const _Float16 *a, const wh_linear *l, void *c, int m, int ldc, int epi, float alpha,
                  bool out16, float *part, int *splits, const HeadsOut *ho, int nho) {
   GemmPlan p = gemm_plan_for(ctx, m, l->cols, l->k);
+  if (p.pipe == PIPE_KW && !l->wt) return wh_fail(ctx, WH_EARG, "gemm: no weight tiles for the k-wavefront kernel");
   if ((p.split > 1 && !part) || nho) p.split = 1;  // packed ranges are written by the tiles' own epilogue
   if (splits) *splits = p.split;
   LdsArgs args{a, l->w, l->bias, p.split > 1 ? (void *)part : c, m, l->rows, l->cols, l->k, l->dual, ldc, epi, alpha,
@@ -1212,6 +1477,9 @@ int launch_lds_t(wh_ctx *ctx, const _Float16 *a, const wh_linear *l, void *c, in
     ProfScope prof(ctx, name, args.skip ? 0.0 : 2.0 * m * l->rows * l->k, args.skip ? 0.0 : bytes);
     const bool sp = p.split > 1;
     bool ok = false;
+    if (p.pipe == PIPE_KW) {
+        if (int rc = kw_launch<WT>(ctx, grid, KwArgs{args, l->wt}, p, out16, &ok)) return rc;
+    }
 #define PLANK(BM, BN, WM, WN, NS, PIPE, WK)                                                                       \
   if (!ok && p.bm == BM && p.bn == BN && p.wm == WM && p.wn == WN && p.ns == NS && p.pipe == PIPE && p.wk == WK) { \
     if (int rc = lds_launch<WT, BM, BN, WM, WN, NS, PIPE, WK>(ctx, grid, args, sp, out16)) return rc;               \

@@ -171,7 +171,14 @@ struct wh_linear {
   size_t row_bytes = 0;
   uint8_t *w = nullptr;
   float *bias = nullptr;  // cols + dual values
+  // The same weights once more in the k-wavefront GEMM's tiles (WTile), in the allocation of w; null for
+  // F32 weights and k % 64 != 0, which that kernel does not take.
+  uint8_t *wt = nullptr;
 };
+// Bytes of a linear layer's weight tiles (0: none), and the kernel that makes them from l->w, on
+// ctx->stream.
+size_t weight_tile_bytes(int type, int rows, int k);
+int launch_weight_tiles(wh_ctx *ctx, const wh_linear *l);
 
 // Sets ctx->error and returns code.
 int wh_fail(wh_ctx *ctx, int code, const char *fmt, ...);

@@ -375,9 +375,9 @@ int wh_tune(wh_ctx *ctx, const char *key, const char *value) {
   if (!strcmp(key, "gemm_plan")) {
     int o[8] = {0, 0, 0, 0, 0, 0, 0, 0};
     if (*v && (sscanf(v, "%d,%d,%d,%d,%d,%d,%d,%d", &o[0], &o[1], &o[2], &o[3], &o[4], &o[5], &o[6], &o[7]) < 6 ||
-               o[5] < 1 || o[5] > 4 || o[7] < 0 || o[7] > 2))
+               o[5] < 1 || o[5] > 4 || o[7] < 0 || o[7] > 16))
       return wh_fail(ctx, WH_EARG,
-                     "wh_tune gemm_plan: \"bm,bn,wm,wn,stages,split[,pipeline[,kgroups]]\" (split 1..4, kgroups 1..2) or \"\"");
+                     "wh_tune gemm_plan: \"bm,bn,wm,wn,stages,split[,pipeline[,kgroups]]\" (split 1..4, kgroups 1..16) or \"\"");
     memcpy(ctx->gemm_plan, o, sizeof o);
   } else if (!strcmp(key, "gemm_shape_plans")) {
     ctx->gemm_shape_plans.clear();
@@ -385,7 +385,7 @@ int wh_tune(wh_ctx *ctx, const char *key, const char *value) {
       std::array<int, 11> o{};
       if (sscanf(q, "%d,%d,%d:%d,%d,%d,%d,%d,%d,%d,%d", &o[0], &o[1], &o[2], &o[3], &o[4], &o[5], &o[6], &o[7], &o[8],
                  &o[9], &o[10]) < 9 ||
-          o[8] < 1 || o[8] > 4 || o[10] < 0 || o[10] > 2)
+          o[8] < 1 || o[8] > 4 || o[10] < 0 || o[10] > 16)
         return wh_fail(ctx, WH_EARG,
                        "wh_tune gemm_shape_plans: \"m,cols,k:bm,bn,wm,wn,stages,split[,pipeline[,kgroups]];...\"");
       ctx->gemm_shape_plans.push_back(o);
@@ -625,7 +625,12 @@ int linear_new(wh_ctx *ctx, const wh_tensor *ws, int count, const float *bias, i
   (void)hipSetDevice(ctx->device);
   size_t wbytes = l->row_bytes * rows;
   // 256 bytes of slack: the GEMM's loaders read whole dwords of the last row.
-  hipError_t e = hipMalloc(&l->w, wbytes + 256);
+  // Then, on a 256-byte boundary, the weight tiles: as many bytes again, made once, so that the GEMMs of
+  // few tiles load whole lines of W straight into registers (rows as stored, 68 bytes of a row per step,
+  // would take a lane 5 loads of 4-byte alignment instead of 2 of 16 bytes).
+  const size_t tiles = weight_tile_bytes(dtype, rows, kp), at_tiles = (wbytes + 256 + 255) / 256 * 256;
+  hipError_t e = hipMalloc(&l->w, tiles ? at_tiles + tiles : wbytes + 256);
+  if (e == hipSuccess && tiles) l->wt = l->w + at_tiles;
   if (e == hipSuccess) e = hipMalloc(&l->bias, sizeof(float) * (size_t)(n > cols + dual ? n : cols + dual));
   if (e != hipSuccess) {
     (void)hipGetLastError();
@@ -654,6 +659,7 @@ int linear_new(wh_ctx *ctx, const wh_tensor *ws, int count, const float *bias, i
   if (rc == WH_OK) rc = stage_upload(ctx, l->w + wbytes, zeros, sizeof zeros);
   if (rc == WH_OK) rc = stage_upload(ctx, l->bias, pb.data(), sizeof(float) * pb.size());
   if (rc == WH_OK) rc = stage_fence(ctx);
+  if (rc == WH_OK && l->wt) rc = launch_weight_tiles(ctx, l);
   if (rc != WH_OK) {
     (void)stage_wait(ctx);
     wh_linear_free(ctx, l);
