@@ -1,17 +1,20 @@
 // The quantized GEMM of Pass::gemm (src/gpu/mod.rs:1394-1426) on gfx950 matrix cores:
 //   c[m][j] = epi(Σ_k h(a[m][k]) · h(W[j][k]) + bias[j]),  h = round to f16 (RNE), f32 accumulate,
 // as gemm.wgsl:170-242 and the CPU backend (src/cpu/gemm.rs:126-177) define it.  W stays in HBM as
-// the GGUF stores it (src/gguf.rs:14-38): Q8_0 34-byte blocks (f16 scale + 32 int8), Q4_0 18-byte
-// blocks (f16 scale + 16 bytes of nibbles), F16 or F32 rows.
+// the GGUF stores it (src/gguf.rs:14-38; the GEMVs read it so): Q8_0 34-byte blocks (f16 scale + 32 int8),
+// Q4_0 18-byte blocks (f16 scale + 16 bytes of nibbles), F16 or F32 rows; and once more in tiles of 32 rows
+// × 64 k in the order the matrix-core lanes load them (WTile, weight_tiles_kernel), for the kernels here.
 //
-// Main kernel (gemm_lds_kernel; k % 64 == 0, W in Q8_0 / Q4_0 / F16, `a` in f16): two LDS stages
-// fed by the LDS DMA of gfx950 — per 64- or 128-wide k step, the a tile (16-byte
-// global_load_lds_dwordx4) and each W row's GGUF blocks as stored (68 or 36 bytes per block pair,
-// 4-byte global_load_lds_dword; F16 rows like a) — so the next step's bytes land while the MFMAs
-// work on the current one.  Each lane dequantizes one block of its W row from LDS into the f16
-// operand of v_mfma_f32_32x32x16_f16: int8 q becomes the f16 1024 + (q + 128) by byte placement, an
-// exact subtraction gives q, and one packed f16 multiply by the block scale rounds q·d once to
-// nearest even — f16(q·d), the reference's exact rounding (products q·d have at most 19 significant
+// Main kernel (gemm_lds_kernel; k % 64 == 0, W in Q8_0 / Q4_0 / F16, `a` in f16): a ring of LDS stages
+// fed by the LDS DMA of gfx950 — per 64- or 128-wide k step, the a tile and W's tiles, all in 16-byte
+// global_load_lds_dwordx4 of whole lines — so the next steps' bytes land while the MFMAs work on the
+// current one.  (W's rows as the GGUF stores them, 68 or 36 bytes of a row per step from 4-byte aligned
+// addresses, cost the loads' address path about twice the cycles and each lane 8 LDS reads of 8 bytes
+// instead of 2 of 16: 750×4096×1024 13.3 -> 12.0 µs, 11616×4096×1024 125.2 -> 115.6 µs, the 60 s Parakeet
+// call 3.94 -> 3.69 ms, 16 windows 23.8 -> 22.5 ms.)  Each lane dequantizes its 8 weights of a substep into
+// the f16 operand of v_mfma_f32_32x32x16_f16: exact conversions of q (int8 by sub-dword conversions, a
+// nibble n as the f16 1024 + n less 1032), then one packed f16 multiply by the block scale rounds q·d once
+// to nearest even — f16(q·d), the reference's exact rounding (products q·d have at most 19 significant
 // bits, so f32 and the f16 multiply round the same value).  The epilogues of Epilogue::params
 // (src/gpu/mod.rs:445-455; gemm.wgsl:72-94) and the dual outputs are fused into the store, in f32
 // or, for a consumer that rounds its input to f16 anyway (another GEMM), in f16.  Shapes with too

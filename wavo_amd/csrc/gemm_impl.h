@@ -293,12 +293,6 @@ __device__ __forceinline__ void dma4s(const void *base, uint32_t off, uint32_t l
   asm volatile("s_nop 0\n\tglobal_load_lds_dword %0, %1" ::"v"(off), "s"(base), "{m0}"(lds) : "memory");
 }
 
-// Two f16 values 1024 + byte0, 1024 + byte1 of x (bytes 0-1, or 2-3 with HI).
-template <bool HI>
-__device__ __forceinline__ half2 magic_pair(uint32_t x) {
-  return __builtin_bit_cast(half2, __builtin_amdgcn_perm(0x64646464u, x, HI ? 0x04030402u : 0x04010400u));
-}
-
 // Two int8 of x (bytes 0-1, or 2-3 with HI) as two f16 (exact: |q| ≤ 128), by sub-dword operand
 // selection of the conversion itself (SDWA: sign-extended byte in, one half of the result out).
 template <bool HI>
@@ -315,69 +309,59 @@ __device__ __forceinline__ half2 i8_pair(uint32_t x) {
   return __builtin_bit_cast(half2, r);
 }
 
-// Q8_0 MFMA fragment of substep S: elements 16·(S % 2) + 8g .. + 8 of block S / 2 of the lane's W
-// row pair, f16(q·d) — the exact conversion of q, then one packed f16 multiply by the block scale.
-// w = the lane's dwords (read_w): for block 0 (data from byte 2 of the pair) three dwords per
-// substep holding the elements from byte 2, for block 1 (data from byte 36) two aligned dwords.
-template <int S>
-__device__ __forceinline__ half8 dequant_q8(const uint32_t *w, half2 d2) {
-  half2 p[4];
-  if constexpr (S < 2) {
-    const uint32_t *x = w + 3 * S;
-    p[0] = i8_pair<true>(x[0]), p[1] = i8_pair<false>(x[1]), p[2] = i8_pair<true>(x[1]), p[3] = i8_pair<false>(x[2]);
-  } else {
-    const uint32_t *x = w + 6 + 2 * (S - 2);
-    p[0] = i8_pair<false>(x[0]), p[1] = i8_pair<true>(x[0]), p[2] = i8_pair<false>(x[1]), p[3] = i8_pair<true>(x[1]);
-  }
-  half8 f;
-#pragma unroll
-  for (int h = 0; h < 4; h++) {
-    const half2 v = p[h] * d2;
-    f[2 * h] = v[0], f[2 * h + 1] = v[1];
-  }
-  return f;
-}
-
-// The MFMA fragment of substep s (elements 8s .. 8s + 7) of one block.  dw = the block's data
-// dwords as read from LDS at the lane's offset, `sh` = bytes of that offset before the data (2 for
-// the even block of a pair: data from byte 2; 0 for the odd one: data dword-aligned), d2 = the
-// block's scale twice.
+// W as the k-wavefront kernel reads it (wh_linear::wt, made from the GGUF bytes when the weights are
+// created): tiles of 32 rows × 64 k, [row tile][k step], rows past the last one zeros.  A tile holds the
+// MFMA operand bytes of lane l = 32g + r (row r, k half g) in the order the lanes load them, 16 bytes per
+// lane and load, so a load is 1 KiB of consecutive bytes:
+//   Q8_0  load i: block i's elements 8g .. 8g + 7, then 16 + 8g .. 16 + 8g + 7 (substeps 2i and 2i + 1);
+//   Q4_0  one load, dword s: substep s's 8 nibbles, element 2h at bits 4h, element 2h + 1 at bits 16 + 4h;
+//   F16   load s: substep s's 8 halves;
+// then, quantized, the two block scales of each row (f16 pairs).  The bytes are as many as in the file.
 template <int WT>
-__device__ __forceinline__ half8 dequant_frag(const uint32_t *dw, uint32_t sh, half2 d2, int s) {
-  half8 f;
-  if constexpr (WT == WH_Q8_0) {
-    const half2 bias = {(_Float16)1152.0f, (_Float16)1152.0f};  // 1024 + 128
-#pragma unroll
-    for (int h = 0; h < 2; h++) {
-      const uint32_t x = __builtin_amdgcn_alignbyte(dw[2 * s + h + 1], dw[2 * s + h], sh) ^ 0x80808080u;
-      const half2 p0 = (magic_pair<false>(x) - bias) * d2, p1 = (magic_pair<true>(x) - bias) * d2;
-      f[4 * h] = p0[0], f[4 * h + 1] = p0[1], f[4 * h + 2] = p1[0], f[4 * h + 3] = p1[1];
-    }
+struct WTile {
+  static constexpr int LOADS = WT == WH_Q8_0 ? 2 : WT == WH_Q4_0 ? 1 : 4;
+  static constexpr int DATA = 1024 * LOADS;
+  static constexpr int BYTES = DATA + (WT == WH_F16 ? 0 : 128);
+};
+
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+
+// The MFMA operand of substep S from a lane's loads of a tile: f16(q·d), as dequant_q8 / dequant_frag.
+template <int WT, int S>
+__device__ __forceinline__ half8 tile_frag(const u32x4 (&q)[WTile<WT>::LOADS], uint32_t sc) {
+  if constexpr (WT == WH_F16) {
+    return __builtin_bit_cast(half8, q[S]);
   } else {
-    // ggml block_q4_0: element i < 16 is the low nibble of byte i, 16 + i the high one; value
-    // (nibble − 8)·d.  Substeps 0-1 take low nibbles of bytes 0-15, substeps 2-3 high ones.
-    const half2 bias = {(_Float16)1032.0f, (_Float16)1032.0f};  // 1024 + 8
+    const half2 sv = __builtin_bit_cast(half2, sc);
+    const half2 d2 = {sv[S / 2], sv[S / 2]};
+    half2 p[4];
+    if constexpr (WT == WH_Q8_0) {
+      const uint32_t x0 = q[S / 2][2 * (S & 1)], x1 = q[S / 2][2 * (S & 1) + 1];
+      p[0] = i8_pair<false>(x0), p[1] = i8_pair<true>(x0), p[2] = i8_pair<false>(x1), p[3] = i8_pair<true>(x1);
+    } else {
+      const half2 bias = {(_Float16)1032.0f, (_Float16)1032.0f};  // 1024 + 8
 #pragma unroll
-    for (int h = 0; h < 2; h++) {
-      const int q = 2 * (s & 1) + h;
-      const uint32_t x = __builtin_amdgcn_alignbyte(dw[q + 1], dw[q], sh);
-      const uint32_t nib = s < 2 ? x & 0x0f0f0f0fu : (x >> 4) & 0x0f0f0f0fu;
-      const half2 p0 = (magic_pair<false>(nib) - bias) * d2, p1 = (magic_pair<true>(nib) - bias) * d2;
-      f[4 * h] = p0[0], f[4 * h + 1] = p0[1], f[4 * h + 2] = p1[0], f[4 * h + 3] = p1[1];
+      for (int h = 0; h < 4; h++)
+        p[h] = __builtin_bit_cast(half2, ((q[0][S] >> (4 * h)) & 0x000f000fu) | 0x64006400u) - bias;
     }
+    half8 f;
+#pragma unroll
+    for (int h = 0; h < 4; h++) {
+      const half2 v = p[h] * d2;
+      f[2 * h] = v[0], f[2 * h + 1] = v[1];
+    }
+    return f;
   }
-  return f;
 }
 
 // Work of one gemm_lds_kernel launch.
 struct LdsArgs {
   const _Float16 *a;
-  const uint8_t *w;
+  const uint8_t *w;  // in tiles (WTile)
   const float *bias;
   void *c;          // output, or f32 partial sums [split][m][cols] with SPLIT
   int m, rows, cols, k, dual, ldc, epi;
   float alpha;
-  size_t row_bytes;
   HeadsOut ho[2];  // column ranges written in attention's packed layout instead of into c (f16 outputs)
   int nho;
   // Non-null: the launch does nothing when *skip == skip_val (c already holds this product: an
@@ -736,11 +720,10 @@ __device__ __forceinline__ void store_c_tile(const LdsArgs &P, const float *cl, 
 // ~16 cycles whatever its width, so W rows move in 16-byte chunks too).
 //
 // LDS layout: the a stages (rows of 8 16-byte chunks, chunk c of row r at (c + r/2) % 8 — the 16
-// lanes that LDS serves together read 16 rows and hit all 64 banks once), then the W stages: F16
-// rows like a, or quantized rows of one block pair (68 or 36 bytes, as stored) in LDS rows of 80 or
-// 48 bytes (whole 16-byte chunks from the pair's start).  At substep s, the
-// lane of MFMA column n and k half g takes k slots 32g + 8s .. + 8 — block g of its W row's pair —
-// and the a fragments the same slots.
+// lanes that LDS serves together read 16 rows and hit all 64 banks once), then the W stages: the tiles'
+// loads as they lie in memory (WTile), each lane reading back its own 16 bytes.  At substep s, the lane
+// of MFMA column n and k half g takes k slots 16s + 8g .. + 8 of its W row, and the a fragments the same
+// slots.
 //
 // Epilogue.  The accumulators go through LDS (f32, rows padded so the two lane halves of a tile hit
 // distinct banks) and leave as 8 consecutive columns per lane: 16-byte loads of c for the residual
@@ -754,18 +737,17 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void gemm_lds_kernel(LdsArgs P) 
   static_assert(WK == 1 || (WK == 2 && PIPE == 0), "k groups in the plain loop");
   constexpr int TM = BM / WM / 32, TN = BN / WN / 32;
   static_assert(TM >= 1 && TN >= 1, "32×32 MFMA tiles per wave");
-  constexpr int PAIR1 = WT == WH_Q8_0 ? 68 : WT == WH_Q4_0 ? 36 : 128;  // W bytes of 64 weights
-  constexpr bool WCH = WT == WH_F16;                                     // W moves in 16-byte chunks
-  // A quantized W row's block pair moves as whole 16-byte chunks from its (4-byte aligned) start: 5
-  // chunks (80 LDS bytes) for Q8_0, 3 (48) for Q4_0; the bytes past the pair are the next pair's (or
-  // the allocation's tail slack) and are never read.  F16 rows move like a.
-  constexpr int WROW = WCH ? 128 : (PAIR1 + 15) / 16 * 16, WCK = WROW / 16;  // LDS bytes, chunks per W row
+  // W's tiles (32 columns × 64 k) as stored: their data, 1 KiB per load, then the scales of up to 8 tiles
+  // in one KiB.
+  constexpr int WL = WTile<WT>::LOADS, WT1 = BN / 32;  // loads per tile, tiles per sub-stage
+  constexpr bool WSC = WT != WH_F16;
+  static_assert(WT1 <= 8, "the scales of a sub-stage in one load");
   // A ring slot holds WK consecutive 64-wide k steps (sub-stages): the a tile's, then the W rows'.
-  constexpr int A_ST0 = BM * 128, W_ST0 = BN * WROW;
+  constexpr int A_ST0 = BM * 128, W_SC0 = WT1 * WTile<WT>::DATA, W_ST0 = W_SC0 + (WSC ? 1024 : 0);
   constexpr int A_ST = WK * A_ST0, W_ST = WK * W_ST0, ST = A_ST + W_ST;
   constexpr int CROW = BN + 8;                                           // f32 per epilogue LDS row
   // NSQ slots asked for, as many as fit in the 160 KiB of LDS.
-  constexpr int NS = NSQ * ST + 16 <= 160 * 1024 ? NSQ : (160 * 1024 - 16) / ST;
+  constexpr int NS = NSQ * ST <= 160 * 1024 ? NSQ : 160 * 1024 / ST;
   static_assert(NS >= 2, "at least two slots");
   static_assert(A_ST0 % 1024 == 0 && W_ST0 % 1024 == 0, "whole DMA instructions per sub-stage");
   constexpr int W_RG = NS * A_ST;                               // the W stages follow the a stages
@@ -780,8 +762,7 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void gemm_lds_kernel(LdsArgs P) 
   // wavefront's last m stages (and at most a few of their instructions besides).
   constexpr int PA = (NIA + NWA - 1) / NWA, PW = (NIW + NWI - 1) / NWI, PI = NIA / NWA + NIW / NWI;
   static_assert((NS - 1) * PI < 64, "vmcnt holds the DMA of NS - 1 steps");
-  // (+16: the odd block of the last W row reads one dword past its row, unused)
-  constexpr int RING = NS * ST + 16;
+  constexpr int RING = NS * ST;
   // Epilogue passes: PG of each wavefront's TM 32-row tiles at a time, the most that fit in the ring
   // (the whole tile when it fits).
   // (k groups: one plane of the pass per group)
@@ -832,25 +813,21 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void gemm_lds_kernel(LdsArgs P) 
     aoff[i] = (uint32_t)(((size_t)min(m0 + r, m - 1) * k + 8 * lc) * 2 + 128 * sub);
     alds[i] = 1024 * n;
   }
+  // (W tiles past the last one are clamped likewise)
+  constexpr int WB = WTile<WT>::BYTES;
+  const int nall = k / 64, wt0 = n0 / 32, wtl = (rows + 31) / 32 - 1;  // k steps per row of tiles, the first tile, the last
   uint32_t woff[PW], wlds[PW];
 #pragma unroll
   for (int i = 0; i < PW; i++) {
     const int n = (wi + NWI * i) % NIW, sub = n / (W_ST0 / 1024), nn = n % (W_ST0 / 1024);
-    if constexpr (WCH) {
-      const int r = 8 * nn + lane / 8, lc = ((lane % 8) - (r >> 1)) & 7;
-      woff[i] = (uint32_t)((size_t)min(n0 + r, rows - 1) * P.row_bytes + 16 * lc + PAIR1 * sub);
-      wlds[i] = 1024 * n;
-    } else {
-      // (Q8_0: rows 16-31 of each 32-row block start 8 bytes into their LDS row, see read_w; a
-      // clamped row 0 — a one-row W, never read — is not moved, as nothing precedes it)
-      const int t = 64 * nn + lane, r = t / WCK, c = t % WCK, row = min(n0 + r, rows - 1);
-      const int shift = WT == WH_Q8_0 && (r & 16) && row > 0 ? 8 : 0;
-      woff[i] = (uint32_t)((size_t)row * P.row_bytes + 16 * c + PAIR1 * sub - shift);
-      wlds[i] = 1024 * n;
-    }
+    const bool data = nn < WT1 * WL;  // else the scales: 8 lanes per tile
+    const int j = data ? nn / WL : min(lane / 8, WT1 - 1);
+    woff[i] = (uint32_t)(((size_t)min(wt0 + j, wtl) * nall + sub) * WB +
+                         (data ? 1024 * (nn % WL) + 16 * lane : WTile<WT>::DATA + 16 * (lane % 8)));
+    wlds[i] = 1024 * n;
   }
   const uint8_t *abase = (const uint8_t *)P.a + (size_t)kb * 128 * WK;
-  const uint8_t *wbase = P.w + (size_t)kb * PAIR1 * WK;
+  const uint8_t *wbase = P.w + (size_t)kb * WB * WK;
   const uint32_t lds0 = lds_addr(lds);
   auto issue_a = [&](int kt, int slot) {
     const uint8_t *ab = abase + (size_t)kt * 128 * WK;
@@ -859,7 +836,7 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void gemm_lds_kernel(LdsArgs P) 
       if (NIA % NWA == 0 || i < NIA / NWA || wave + NWA * i < NIA) dma16s(ab, aoff[i], lds0 + slot * A_ST + alds[i]);
   };
   auto issue_w = [&](int kt, int slot) {
-    const uint8_t *wb = wbase + (size_t)kt * PAIR1 * WK;
+    const uint8_t *wb = wbase + (size_t)kt * WB * WK;
 #pragma unroll
     for (int i = 0; i < PW; i++)
       if (NIW % NWI == 0 || i < NIW / NWI || wi + NWI * i < NIW) dma16s(wb, woff[i], lds0 + W_RG + slot * W_ST + wlds[i]);
@@ -869,68 +846,25 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void gemm_lds_kernel(LdsArgs P) 
     issue_w(kt, slot);
   };
 
-  // The lane's k chunk (of 8 in a step) at substep s.  Q8_0: 2s + g — block s/2 of the pair at
-  // every lane of a substep, so the bytes of a substep sit at the same place in every lane's dwords;
-  // Q4_0 and F16: 4g + s — block g.  a and W fragments take the same chunk.
-  constexpr bool Q8 = WT == WH_Q8_0;
-  auto chunk = [&](int s) { return Q8 ? 2 * s + g : 4 * g + s; };
-  // LDS read offsets of the lane: a chunk of row wm + lrow (+32i), rotated by row/2; the lane's W
-  // dwords (Q8_0: from byte 8g of its row pair, the scales in dwords 0 and 8 of the row; Q4_0:
-  // g = 0 reads dwords 0.. with the data from byte 2, g = 1 the dwords from byte BLK + 2 with the
-  // scale in the high half of the dword before); F16 chunks like a.
+  // The lane's k chunk (of 8 in a step) at substep s is 2s + g.  LDS read offsets of the lane: the a chunk
+  // of row wm + lrow (+32i), rotated by row/2; its 16 bytes of each load of its W tiles, and the scales of
+  // its row.
   uint32_t a_off[4];
 #pragma unroll
-  for (int s = 0; s < 4; s++) a_off[s] = kg * A_ST0 + (wm + lrow) * 128 + 16 * ((chunk(s) + (lrow >> 1)) & 7);
-  constexpr int ND = Q8 ? 10 : WT == WH_Q4_0 ? 5 : 16;  // dwords per lane per W row and step
-  constexpr int NSC = Q8 ? 2 : 1;                       // scale dwords per lane per W row and step
-  constexpr int BLK = PAIR1 / 2;
-  const uint32_t w_row = W_RG + kg * W_ST0 + (wn + lrow) * WROW + (Q8 ? 8 * ((lrow >> 4) & 1) : 0);
-  const uint32_t w_dat = Q8 ? w_row + 8 * g : w_row + (g ? BLK + 2 : 0), w_sc = w_row + (g ? BLK - 2 : 0);
-  uint32_t wf_off[4];
-#pragma unroll
-  for (int s = 0; s < 4; s++) wf_off[s] = w_row + 16 * ((chunk(s) + (lrow >> 1)) & 7);
+  for (int s = 0; s < 4; s++) a_off[s] = kg * A_ST0 + (wm + lrow) * 128 + 16 * ((2 * s + g + (lrow >> 1)) & 7);
+  const uint32_t w_dat = W_RG + kg * W_ST0 + (wn / 32) * WTile<WT>::DATA + 16 * lane;
+  const uint32_t w_sc = W_RG + kg * W_ST0 + W_SC0 + (wn / 32) * 128 + 4 * lrow;
 
   auto read_a = [&](half8 (&f)[TM], int slot, int s) {
 #pragma unroll
     for (int i = 0; i < TM; i++) f[i] = *(const half8 *)(lds + a_off[s] + slot * A_ST + i * 4096);
   };
-  auto read_w = [&](uint32_t (&w)[TN][ND], uint32_t (&sc)[TN][NSC], int slot) {
+  auto read_w = [&](u32x4 (&w)[TN][WL], uint32_t (&sc)[TN], int slot) {
 #pragma unroll
     for (int j = 0; j < TN; j++) {
-      if constexpr (WCH) {
 #pragma unroll
-        for (int s = 0; s < 4; s++) {
-          const uint4 x = *(const uint4 *)(lds + wf_off[s] + slot * W_ST + j * 32 * WROW);
-          w[j][4 * s] = x.x, w[j][4 * s + 1] = x.y, w[j][4 * s + 2] = x.z, w[j][4 * s + 3] = x.w;
-        }
-        sc[j][0] = 0;
-      } else if constexpr (Q8) {
-        // Pair bytes 2 + 8g .. (block 0, substeps 0-1: dwords 0-2 and 4-6 from byte 8g) and
-        // 36 + 8g .. (block 1, substeps 2-3: dwords 9-10 and 13-14), read as the 16 dwords from byte
-        // 8g in 8-byte reads: with 80-byte LDS rows, rows r and r + 16 of a 32-row block would share
-        // banks, so rows 16-31 sit 8 bytes further into their LDS row (measured on gfx950: single
-        // dwords from the rows as stored cost 6 bank-conflict cycles per read, 8-byte reads from the
-        // moved rows none).  The scales at bytes 0 and 34: dword 0 of lane group 0's span (lanes
-        // 32-63 take it from lane − 32) and dword 8 − 2g.
-        const uint2 *q = (const uint2 *)(lds + w_dat + slot * W_ST + j * 32 * WROW);
-        uint32_t d[16];
-#pragma unroll
-        for (int i = 0; i < 8; i++) {
-          const uint2 v = q[i];
-          d[2 * i] = v.x, d[2 * i + 1] = v.y;
-        }
-        constexpr int at[10] = {0, 1, 2, 4, 5, 6, 9, 10, 13, 14};
-#pragma unroll
-        for (int i = 0; i < 10; i++) w[j][i] = d[at[i]];
-        uint32_t s0 = d[0], s0b = d[0];
-        xlane::swap32(s0, s0b);  // lanes 32-63: lane − 32's dword 0
-        sc[j][0] = s0, sc[j][1] = g ? d[6] : d[8];
-      } else {
-        const uint32_t *q = (const uint32_t *)(lds + w_dat + slot * W_ST + j * 32 * WROW);
-#pragma unroll
-        for (int i = 0; i < ND; i++) w[j][i] = q[i];
-        sc[j][0] = *(const uint32_t *)(lds + w_sc + slot * W_ST + j * 32 * WROW);
-      }
+      for (int i = 0; i < WL; i++) w[j][i] = *(const u32x4 *)(lds + w_dat + slot * W_ST + j * WTile<WT>::DATA + 1024 * i);
+      sc[j] = WSC ? *(const uint32_t *)(lds + w_sc + slot * W_ST + 128 * j) : 0u;
     }
   };
 
@@ -939,20 +873,9 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void gemm_lds_kernel(LdsArgs P) 
   for (int i = 0; i < TM; i++)
 #pragma unroll
     for (int j = 0; j < TN; j++) acc[i][j] = floatx16{};
-  const uint32_t sh = g ? 0u : 2u;
-  // The MFMA operand of W column block j at substep s: f16 chunks as read (F16), or the lane's
-  // quantized dwords dequantized (f16(q·d)).
-  auto wfrag = [&](const uint32_t (&w)[TN][ND], const uint32_t (&scl)[TN][NSC], int j, auto s_c) -> half8 {
-    constexpr int s = decltype(s_c)::value;
-    if constexpr (WCH) return __builtin_bit_cast(half8, make_uint4(w[j][4 * s], w[j][4 * s + 1], w[j][4 * s + 2], w[j][4 * s + 3]));
-    else if constexpr (Q8) {
-      const half2 sv = __builtin_bit_cast(half2, scl[j][s >> 1]);  // block 0: low half; block 1: high
-      const _Float16 d = s < 2 ? sv[0] : sv[1];
-      return dequant_q8<s>(w[j], half2{d, d});
-    } else {
-      const _Float16 d = __builtin_bit_cast(_Float16, (uint16_t)(g ? scl[j][0] >> 16 : scl[j][0] & 0xffffu));
-      return dequant_frag<WT>(w[j], sh, half2{d, d}, s);
-    }
+  // The MFMA operand of W column block j at substep s (f16(q·d), or the f16 weights).
+  auto wfrag = [&](const u32x4 (&w)[TN][WL], const uint32_t (&scl)[TN], int j, auto s_c) -> half8 {
+    return tile_frag<WT, decltype(s_c)::value>(w[j], scl[j]);
   };
   if constexpr (PIPE == 2) {
     // Ping-pong.  Two groups of four wavefronts (group 1 = waves 4-7; a workgroup's wavefronts go to
@@ -970,7 +893,8 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void gemm_lds_kernel(LdsArgs P) 
     static_assert(NIA % NW == 0 && NIA / NW <= 4, "at most one a-tile DMA instruction per wavefront and substep");
     const bool g1 = wave >= 4;
     constexpr int QA = NIA / NW, QW = NIW / 4;  // DMA instructions per wavefront and stage (W: the fewest)
-    uint32_t wq[TN][ND], sc[TN][NSC];
+    u32x4 wq[TN][WL];
+    uint32_t sc[TN];
     half8 af[2][TM], wf[4][TN];
     // The MFMAs of substep s; a-tile DMA instruction s of stage kd (if any) after the first.
     auto mm = [&](const half8 (&f)[TM], const half8 (&b)[TN], const uint8_t *ab, int slot_d, auto s_c) {
@@ -1048,10 +972,11 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void gemm_lds_kernel(LdsArgs P) 
 #pragma unroll
     for (int s = 0; s < NS; s++)
       if (s < nk) issue(s, s);
-    uint32_t wq[2][TN][ND], sc[2][TN][NSC];
+    u32x4 wq[2][TN][WL];
+    uint32_t sc[2][TN];
     half8 af[2][TM];
     // Substep s of a step: dequantize the lane's W fragment (quantized) and run the TM × TN MFMAs.
-    auto mma = [&](const half8 (&f)[TM], const uint32_t (&w)[TN][ND], const uint32_t (&scl)[TN][NSC], auto s_c) {
+    auto mma = [&](const half8 (&f)[TM], const u32x4 (&w)[TN][WL], const uint32_t (&scl)[TN], auto s_c) {
 #pragma unroll
       for (int j = 0; j < TN; j++) {
         const half8 b = wfrag(w, scl, j, s_c);
@@ -1153,55 +1078,6 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void gemm_lds_kernel(LdsArgs P) 
 
 // ------------------------------------------------------------------- wavefronts splitting k
 
-// W as the k-wavefront kernel reads it (wh_linear::wt, made from the GGUF bytes when the weights are
-// created): tiles of 32 rows × 64 k, [row tile][k step], rows past the last one zeros.  A tile holds the
-// MFMA operand bytes of lane l = 32g + r (row r, k half g) in the order the lanes load them, 16 bytes per
-// lane and load, so a load is 1 KiB of consecutive bytes:
-//   Q8_0  load i: block i's elements 8g .. 8g + 7, then 16 + 8g .. 16 + 8g + 7 (substeps 2i and 2i + 1);
-//   Q4_0  one load, dword s: substep s's 8 nibbles, element 2h at bits 4h, element 2h + 1 at bits 16 + 4h;
-//   F16   load s: substep s's 8 halves;
-// then, quantized, the two block scales of each row (f16 pairs).  The bytes are as many as in the file.
-template <int WT>
-struct WTile {
-  static constexpr int LOADS = WT == WH_Q8_0 ? 2 : WT == WH_Q4_0 ? 1 : 4;
-  static constexpr int DATA = 1024 * LOADS;
-  static constexpr int BYTES = DATA + (WT == WH_F16 ? 0 : 128);
-};
-
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-
-// The MFMA operand of substep S from a lane's loads of a tile: f16(q·d), as dequant_q8 / dequant_frag.
-template <int WT, int S>
-__device__ __forceinline__ half8 tile_frag(const u32x4 (&q)[WTile<WT>::LOADS], uint32_t sc) {
-  if constexpr (WT == WH_F16) {
-    return __builtin_bit_cast(half8, q[S]);
-  } else {
-    const half2 sv = __builtin_bit_cast(half2, sc);
-    const half2 d2 = {sv[S / 2], sv[S / 2]};
-    half2 p[4];
-    if constexpr (WT == WH_Q8_0) {
-      const uint32_t x0 = q[S / 2][2 * (S & 1)], x1 = q[S / 2][2 * (S & 1) + 1];
-      p[0] = i8_pair<false>(x0), p[1] = i8_pair<true>(x0), p[2] = i8_pair<false>(x1), p[3] = i8_pair<true>(x1);
-    } else {
-      const half2 bias = {(_Float16)1032.0f, (_Float16)1032.0f};  // 1024 + 8
-#pragma unroll
-      for (int h = 0; h < 4; h++)
-        p[h] = __builtin_bit_cast(half2, ((q[0][S] >> (4 * h)) & 0x000f000fu) | 0x64006400u) - bias;
-    }
-    half8 f;
-#pragma unroll
-    for (int h = 0; h < 4; h++) {
-      const half2 v = p[h] * d2;
-      f[2 * h] = v[0], f[2 * h + 1] = v[1];
-    }
-    return f;
-  }
-}
-
-struct KwArgs : LdsArgs {
-  const uint8_t *wt;  // W in tiles (WTile)
-};
-
 // c tile (32·TM) × (32·TN) per workgroup of WK wavefronts, each over its own 1/WK of the k steps (for
 // the whole tile): GEMMs of few tiles, whose time is the latency of a workgroup's chain of steps rather
 // than any throughput.  A wavefront shares nothing with the others until the end: it loads its a rows
@@ -1213,7 +1089,7 @@ struct KwArgs : LdsArgs {
 // 275×768×3072 13.8 (two splits and their finish) -> 7.6, 25×1024×1024 7.6 -> 4.3, 500×2048×1024
 // 10.1 -> 8.1.  The sums of the WK wavefronts are added in wavefront order through LDS planes.
 template <int WT, int TM, int TN, int WK, bool OUT16>
-__global__ __launch_bounds__(64 * WK) void gemm_kw_kernel(KwArgs P) {
+__global__ __launch_bounds__(64 * WK) void gemm_kw_kernel(LdsArgs P) {
   constexpr int BM = 32 * TM, BN = 32 * TN, NT = 64 * WK, CROW = BN + 8, CPL = BM * CROW;
   constexpr int A_ST = BM * 128;  // LDS bytes of one step's a rows
   constexpr int RING = WK * 2 * A_ST, PLANES = WK * CPL * 4;
@@ -1245,7 +1121,7 @@ __global__ __launch_bounds__(64 * WK) void gemm_kw_kernel(KwArgs P) {
   const uint8_t *wb[TN];
 #pragma unroll
   for (int j = 0; j < TN; j++)
-    wb[j] = P.wt + ((size_t)min(n0 / 32 + j, (P.rows + 31) / 32 - 1) * nkt + k0) * WTile<WT>::BYTES;
+    wb[j] = P.w + ((size_t)min(n0 / 32 + j, (P.rows + 31) / 32 - 1) * nkt + k0) * WTile<WT>::BYTES;
   auto load_a = [&](u32x4 (&r)[NA], int t) {
     const uint8_t *b = ab + (size_t)t * 128;
 #pragma unroll
@@ -1402,8 +1278,7 @@ __global__ __launch_bounds__(256) void split_finish_kernel(const float *__restri
 
 template <int WT, int BM, int BN, int WM, int WN, int NS, int PIPE, int WK>
 int lds_launch(wh_ctx *ctx, dim3 grid, const LdsArgs &a, bool split, bool out16) {
-  constexpr int WROW = WT == WH_Q8_0 ? 80 : WT == WH_Q4_0 ? 48 : 128;  // LDS bytes per W row (the kernel's)
-  if constexpr (PIPE == 2 && (WT == WH_F16 || NS * (BM * 128 + BN * WROW) + 16 > 160 * 1024)) {
+  if constexpr (PIPE == 2 && (WT == WH_F16 || NS * (BM * 128 + BN / 32 * WTile<WT>::DATA + 1024) > 160 * 1024)) {
     // (not built: the ring would exceed the LDS, or F16 rows, which need no dequantization to hide)
     return wh_fail(ctx, WH_EARG, "gemm: no ping-pong kernel for %d slots of a %dx%d tile of this weight type", NS, BM, BN);
   } else {
@@ -1417,7 +1292,7 @@ int lds_launch(wh_ctx *ctx, dim3 grid, const LdsArgs &a, bool split, bool out16)
 
 // The k-wavefront kernel of plan p (*ok: built).
 template <int WT>
-int kw_launch(wh_ctx *ctx, dim3 grid, const KwArgs &a, const GemmPlan &p, bool out16, bool *ok) {
+int kw_launch(wh_ctx *ctx, dim3 grid, const LdsArgs &a, const GemmPlan &p, bool out16, bool *ok) {
 #define KW(TM, TN, WK)                                                                              \
   if (p.bm == 32 * TM && p.bn == 32 * TN && p.wk == WK && p.split == 1) {                           \
     if (out16) wh_launch(ctx, gemm_kw_kernel<WT, TM, TN, WK, true>, grid, 64 * WK, 0, a);           \
@@ -1435,11 +1310,11 @@ template <int WT>
 int launch_lds_t(wh_ctx *ctx, const _Float16 *a, const wh_linear *l, void *c, int m, int ldc, int epi, float alpha,
                  bool out16, float *part, int *splits, const HeadsOut *ho, int nho) {
   GemmPlan p = gemm_plan_for(ctx, m, l->cols, l->k);
-  if (p.pipe == PIPE_KW && !l->wt) return wh_fail(ctx, WH_EARG, "gemm: no weight tiles for the k-wavefront kernel");
+  if (!l->wt) return wh_fail(ctx, WH_EARG, "gemm: a linear layer without weight tiles");
   if ((p.split > 1 && !part) || nho) p.split = 1;  // packed ranges are written by the tiles' own epilogue
   if (splits) *splits = p.split;
-  LdsArgs args{a, l->w, l->bias, p.split > 1 ? (void *)part : c, m, l->rows, l->cols, l->k, l->dual, ldc, epi, alpha,
-               l->row_bytes, {}, nho, nullptr, 0, 1};
+  LdsArgs args{a, l->wt, l->bias, p.split > 1 ? (void *)part : c, m, l->rows, l->cols, l->k, l->dual, ldc, epi, alpha,
+               {}, nho, nullptr, 0, 1};
   // A tagged output (ctx->gemm_skip, set by the caller for this launch): whole-k plans only (a split
   // launch's partial sums are finished by another kernel).
   if (ctx->gemm_skip && p.split == 1) args.skip = ctx->gemm_skip, args.skip_val = ctx->gemm_skip_val;
@@ -1478,7 +1353,7 @@ int launch_lds_t(wh_ctx *ctx, const _Float16 *a, const wh_linear *l, void *c, in
     const bool sp = p.split > 1;
     bool ok = false;
     if (p.pipe == PIPE_KW) {
-        if (int rc = kw_launch<WT>(ctx, grid, KwArgs{args, l->wt}, p, out16, &ok)) return rc;
+        if (int rc = kw_launch<WT>(ctx, grid, args, p, out16, &ok)) return rc;
     }
 #define PLANK(BM, BN, WM, WN, NS, PIPE, WK)                                                                       \
   if (!ok && p.bm == BM && p.bn == BN && p.wm == WM && p.wn == WN && p.ns == NS && p.pipe == PIPE && p.wk == WK) { \

@@ -171,8 +171,8 @@ struct wh_linear {
   size_t row_bytes = 0;
   uint8_t *w = nullptr;
   float *bias = nullptr;  // cols + dual values
-  // The same weights once more in the k-wavefront GEMM's tiles (WTile), in the allocation of w; null for
-  // F32 weights and k % 64 != 0, which that kernel does not take.
+  // The same weights once more in the GEMM kernels' tiles (WTile), in the allocation of w; null for F32
+  // weights and k % 64 != 0, which those kernels do not take.
   uint8_t *wt = nullptr;
 };
 // Bytes of a linear layer's weight tiles (0: none), and the kernel that makes them from l->w, on

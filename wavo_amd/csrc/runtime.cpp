@@ -625,9 +625,8 @@ int linear_new(wh_ctx *ctx, const wh_tensor *ws, int count, const float *bias, i
   (void)hipSetDevice(ctx->device);
   size_t wbytes = l->row_bytes * rows;
   // 256 bytes of slack: the GEMM's loaders read whole dwords of the last row.
-  // Then, on a 256-byte boundary, the weight tiles: as many bytes again, made once, so that the GEMMs of
-  // few tiles load whole lines of W straight into registers (rows as stored, 68 bytes of a row per step,
-  // would take a lane 5 loads of 4-byte alignment instead of 2 of 16 bytes).
+  // Then, on a 256-byte boundary, the weight tiles: as many bytes again, made once, so that the GEMMs load
+  // W in whole lines (see gemm.hip).
   const size_t tiles = weight_tile_bytes(dtype, rows, kp), at_tiles = (wbytes + 256 + 255) / 256 * 256;
   hipError_t e = hipMalloc(&l->w, tiles ? at_tiles + tiles : wbytes + 256);
   if (e == hipSuccess && tiles) l->wt = l->w + at_tiles;
