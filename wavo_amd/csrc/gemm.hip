@@ -85,14 +85,17 @@ GemmPlan gemm_plan_for(const wh_ctx *ctx, int m, int cols, int k) {
     // groups where they divide every split (14.3 against 15.0 µs in the step, the groups' sums in
     // LDS planes of their own).
     p = {96, 64, 1, 2, 2, 4, 0, k % (4 * 128) == 0 ? 2 : 1};
-  else if (t128 * 4 <= 2L * cus && k % (4 * 64) == 0 && k / (4 * 64) >= 16)
-    // The same with up to two workgroups per CU (Whisper's fc2, 1500 × 1280 × 5120: 1.18 + its
-    // finish against 1.82 ms per call for 64×64 tiles whole).
-    p = {128, 128, 2, 2, 2, 4};
-  else if (t64 < cus) {
-    // Split only while every split keeps at least 16 k steps: shorter ones spend more on the
-    // pipeline's fill and the partial sums than the extra workgroups win (k = 1024 runs faster whole).
-    while (p.split < 4 && t64 * p.split < 2L * cus && k % (2 * p.split * 64) == 0 && k / (2 * p.split * 64) >= 16)
+  else if (t128 * 4 <= 2L * cus && k % 128 == 0 && k / (4 * 64) >= 16 &&
+           (long)((cols + 127) / 128) * ((m + 95) / 96) <= cus)
+    // The same over up to half a 128×128 tile per CU (Whisper's fc2, 1500 × 1280 × 5120): the whole k in
+    // two k groups over 96×128 tiles, 160 of them; no partial sums (four layers and their window 638 µs,
+    // against 645 for 128×128 tiles with k split 4 ways, 640 for 96×64 tiles, 676 split 2 ways).
+    p = {96, 128, 1, 4, 3, 1, 0, 2};
+  else if (t64 <= cus) {
+    // Split only while every split keeps at least 32 k steps: shorter ones spend more on the pipeline's
+    // fill, the partial sums and their finish than the extra workgroups win (750 frames of GigaAM, whose
+    // 768 × 3072 projections split in two and finished with the norm: 2 567 µs per call, whole 2 423).
+    while (p.split < 4 && t64 * p.split < 2L * cus && k % (2 * p.split * 64) == 0 && k / (2 * p.split * 64) >= 32)
       p.split *= 2;
     // Unsplit: two k groups of 4 wavefronts over a 4-slot ring (one workgroup per CU; the 750-frame
     // 1024 × 1024 projections 9.5 against 10.0 µs in the step; deeper rings alone are slower there:
@@ -104,21 +107,20 @@ GemmPlan gemm_plan_for(const wh_ctx *ctx, int m, int cols, int k) {
     // in the step for 64×64 tiles; 12.2 with 4 slots).
     p = {96, 64, 1, 2, 2, 1, 0, 2};
   // Few tiles: wavefronts that split k (gemm_kw_kernel), the smallest of its tiles that still run at once
-  // (one workgroup per CU), whose chain of steps is then the shortest.  Both sides inside the encoder
-  // call, µs per call with that one layer on either kernel: 60 Parakeet frames (32×32 tiles, 32×64 for the
-  // wider ones) 2 289 against 2 073 for the 1024 × 1024 projections, 2 298 for 4096 × 1024, all of them
-  // 2 807; 31 GigaAM frames 1 915 against 1 380 all together.  64×64 tiles up to two per CU where 96-row
-  // tiles would not run at once either (500 frames, 4096 × 1024: 3 244 against 3 132), but not past 1024
-  // rows (Whisper's 1500 × 1280 × 1280: 723 against 708 per four layers), and not over a long k, which
-  // the split plans above walk faster (500 frames' 1024 × 4096: 3 400 on 64×64 tiles here, 3 319 split,
-  // 3 132 on 32×64; 750 frames': 4 071 against 3 944).
+  // (one workgroup per CU), whose chain of steps is then the shortest.  µs per encoder call with that one
+  // layer on the LDS-DMA kernel and here: 60 Parakeet frames 2 289 against 2 073 for the 1024 × 1024
+  // projections (32×32 tiles), 2 298 for 4096 × 1024 (32×64), 2 807 for all of them; 275 GigaAM frames
+  // 1 790 against 1 682 for the 768 × 768 ones, 1 854 for 768 × 3072.  With 64×64 tiles the LDS-DMA
+  // kernel's two k groups are the faster ones while the tiles run at once (750 frames' 1024 × 1024: 3 584
+  // against 3 626; 275 frames' 3072 × 1024: 2 846 against 2 886), this kernel for one to two tiles per CU
+  // of few rows (750 frames' 2048 × 1024: 3 630 against 3 605; 500 frames' 3072 × 1024: 3 153 against
+  // 3 105; Whisper's 1500 rows and tiles past two per CU stay above).
   {
     const long t32 = (long)((cols + 31) / 32) * ((m + 31) / 32), t3264 = (long)((cols + 63) / 64) * ((m + 31) / 32);
-    const long t96 = (long)((cols + 63) / 64) * ((m + 95) / 96);
     if ((size_t)m * k < ((size_t)1 << 30)) {  // 32-bit byte offsets into a
       if (t32 <= cus) p = {32, 32, 1, 1, 2, 1, PIPE_KW, 8};
       else if (t3264 <= cus) p = {32, 64, 1, 1, 2, 1, PIPE_KW, 8};
-      else if (k <= 2048 && (t64 <= cus || (m < 1024 && t64 <= 2L * cus && t96 > cus))) p = {64, 64, 1, 1, 2, 1, PIPE_KW, 4};
+      else if (m < 1024 && k <= 2048 && t64 > cus && t64 <= 2L * cus) p = {64, 64, 1, 1, 2, 1, PIPE_KW, 4};
     }
   }
   if (ctx->gemm_plan[0]) {  // tuning override (wh_tune "gemm_plan"): bm, bn, wm, wn, stages, split, pipeline, kgroups
