@@ -515,6 +515,21 @@ def test_relative_attention(gpu, t, heads, hd, valid):
     close(gpu.read(ob, (t, d)), want, tol=ATT_TOL)
 
 
+# The pack launch's parts (K/V blocks, position rows, query rows, 32 rows each) at their edges: rows that
+# end inside a part or on its boundary, head dims below, at and past a padded width of 32, 64 and 128.
+@pytest.mark.parametrize("t", [1, 32, 33])
+@pytest.mark.parametrize("hd", [4, 32, 36, 68, 128])
+def test_attention_pack_edges(gpu, t, hd):
+    heads, d = 3, 3 * hd
+    qkv, pos, u, vb, rows = relative_inputs(t, heads, hd)
+    ob = gpu.buffer(t * d)
+    gpu.attention(gpu.upload(rows), None, gpu.upload(pos), ob, t, heads, hd)
+    close(gpu.read(ob, (t, d)), ox.relative_attention(qkv, pos, u, vb, t, heads, hd, -1), tol=ATT_TOL, what="relative")
+    gpu.attention(gpu.upload(qkv), None, None, ob, t, heads, hd)
+    want = ox.attention(qkv, 3 * d, np.ascontiguousarray(qkv[:, 2 * d:]), d, t, heads, hd)
+    close(gpu.read(ob, (t, d)), want, tol=ATT_TOL, what="plain")
+
+
 @pytest.mark.parametrize("heads", [8, 3])
 @pytest.mark.parametrize("valid", [None, 400])
 def test_relative_attention_many_splits(valid, heads):

@@ -136,6 +136,33 @@ __device__ __forceinline__ int swz(int row) {
 
 // ---------------------------------------------------------------------------------- pack pass
 
+// Four values of a row, f32 or f16 (rows and their parts start on 4 values of 16-byte aligned buffers),
+// rounded to f16.
+__device__ __forceinline__ half4 four(const float *p) {
+  const float4 x = *(const float4 *)p;
+  return half4{(_Float16)x.x, (_Float16)x.y, (_Float16)x.z, (_Float16)x.w};
+}
+__device__ __forceinline__ half4 four(const _Float16 *p) { return *(const half4 *)p; }
+
+// The part of 32 rows from row r0 (of `rows`; hd of their values from `src`, stride floats apart) that this
+// thread takes, zeros past the rows and past hd, 4 values per round: every load issued before the first
+// use, from clamped addresses (one memory round trip, not one per round).
+template <int DP, typename T>
+struct RowPart {
+  static constexpr int N = 32 * DP / 4 / 256;  // rounds
+  half4 x[N];
+  __device__ __forceinline__ static int row(int n) { return ((int)threadIdx.x + 256 * n) / (DP / 4); }
+  __device__ __forceinline__ static int dim(int n) { return 4 * (((int)threadIdx.x + 256 * n) % (DP / 4)); }
+  __device__ __forceinline__ void load(const T *__restrict__ src, long stride, int r0, int rows, int hd) {
+#pragma unroll
+    for (int n = 0; n < N; n++) x[n] = four(src + (long)min(max(r0 + row(n), 0), rows - 1) * stride + min(dim(n), hd - 4));
+  }
+  __device__ __forceinline__ half4 value(int n, int r0, int rows, int hd) const {
+    const int r = r0 + row(n);
+    return r >= 0 && r < rows && dim(n) < hd ? x[n] : half4{};
+  }
+};
+
 // K rows [batch][head][tk][DP] and Vᵀ [batch][head][DP][tk] as f16, zeros past t and hd.  One
 // workgroup per 32 keys of one head.  T = float or _Float16 input.
 template <int DP, typename T>
@@ -144,17 +171,16 @@ __device__ __forceinline__ void pack_kv(const T *__restrict__ k, int ks, long kb
                                         _Float16 *__restrict__ vt, int j0, int head, int b) {
   __shared__ _Float16 tr[KB][DP + 2];
   const size_t off = ((size_t)b * heads + head) * tk * DP;
-  for (int e = threadIdx.x; e < KB * DP / 4; e += 256) {
-    const int key = e / (DP / 4), d = 4 * (e % (DP / 4)), j = j0 + key;
-    half4 kx = {}, vx = {};
-    if (j < t && d < hd) {
-      const T *kr = k + kbs * b + (long)j * ks + head * hd + d, *vr = v + vbs * b + (long)j * vs + head * hd + d;
+  RowPart<DP, T> kx, vx;
+  kx.load(k + kbs * b + head * hd, ks, j0, t, hd);
+  vx.load(v + vbs * b + head * hd, vs, j0, t, hd);
 #pragma unroll
-      for (int q = 0; q < 4; q++) kx[q] = (_Float16)kr[q], vx[q] = (_Float16)vr[q];
-    }
-    *(half4 *)(kp + off + (size_t)j * DP + d) = kx;
+  for (int n = 0; n < RowPart<DP, T>::N; n++) {
+    const int key = kx.row(n), d = kx.dim(n);
+    *(half4 *)(kp + off + (size_t)(j0 + key) * DP + d) = kx.value(n, j0, t, hd);
+    const half4 y = vx.value(n, j0, t, hd);
 #pragma unroll
-    for (int q = 0; q < 4; q++) tr[key][d + q] = vx[q];
+    for (int q = 0; q < 4; q++) tr[key][d + q] = y[q];
   }
   __syncthreads();
   for (int e = threadIdx.x; e < DP * (KB / 8); e += 256) {
@@ -172,29 +198,55 @@ template <int DP, typename T>
 __device__ __forceinline__ void pack_pos(const T *__restrict__ pos, int ps, int prow, int hd, int pfront, int prows,
                                          _Float16 *__restrict__ pp, int x, int head) {
   const size_t off = (size_t)head * prows * DP;
-  for (int e = threadIdx.x; e < 32 * DP / 4; e += 256) {
-    const int sr = x * 32 + e / (DP / 4), d = 4 * (e % (DP / 4)), r = sr - pfront;
-    half4 x = {};
-    if (r >= 0 && r < prow && d < hd) {
-      const T *pr = pos + (long)r * ps + head * hd + d;
+  const int r0 = 32 * x - pfront;
+  RowPart<DP, T> px;
+  px.load(pos + head * hd, ps, r0, prow, hd);
 #pragma unroll
-      for (int q = 0; q < 4; q++) x[q] = (_Float16)pr[q];
-    }
-    *(half4 *)(pp + off + (size_t)sr * DP + d) = x;
+  for (int n = 0; n < RowPart<DP, T>::N; n++)
+    *(half4 *)(pp + off + (size_t)(32 * x + px.row(n)) * DP + px.dim(n)) = px.value(n, r0, prow, hd);
+}
+
+// A head's query rows rounded to f16, [batch · t][heads · hd] (f32 calls: the flash kernel reads f16 rows).
+// One workgroup per 32 queries of one head.
+template <int DP, typename T>
+__device__ __forceinline__ void round_q(const T *__restrict__ q, long qs, int t, int hd, int ch, _Float16 *__restrict__ q16,
+                                        int i0, int head, int b) {
+  RowPart<DP, T> x;
+  x.load(q + (long)b * t * qs + head * hd, qs, i0, t, hd);
+#pragma unroll
+  for (int n = 0; n < RowPart<DP, T>::N; n++) {
+    const int i = i0 + x.row(n), d = x.dim(n);
+    if (i < t && d < hd) *(half4 *)(q16 + ((size_t)b * t + i) * ch + head * hd + d) = x.x[n];
   }
 }
 
-// Both packs in one launch: workgroups x < tk / KB pack K/Vᵀ (window z), the next prows / 32 (window
-// 0 only) the position rows.
+// The query rows of an f32 call and their f16 copies: q (q + u) and, with relative positions, q + v.
+struct Queries {
+  const float *q, *qv;
+  _Float16 *q16, *qv16;
+  int qs;
+};
+
+// All packs in one launch: workgroups x < tk / KB pack K/Vᵀ (window z), the next prows / 32 (window 0 only)
+// the position rows, then, f32 input, 32 query rows each and their q + v rows.  Bound by the memory round
+// trips of a workgroup and by the launch: with the queries rounded by a launch of their own, which also
+// read and wrote the K and V columns, and a round trip per 256 loads of a part, the whole call took 31.0 µs
+// for 750 × 8 × 128 relative f32 rows; in one launch with each part's loads together 26.9.
 template <int DP, typename T>
 __global__ __launch_bounds__(256) void pack_kernel(const T *__restrict__ k, int ks, long kbs, const T *__restrict__ v,
                                                    int vs, long vbs, int t, int heads, int hd, int tk,
                                                    _Float16 *__restrict__ kp, _Float16 *__restrict__ vt,
                                                    const T *__restrict__ pos, int ps, int prow, int pfront, int prows,
-                                                   _Float16 *__restrict__ pp) {
-  const int nkv = tk / KB;
-  if ((int)blockIdx.x < nkv) pack_kv<DP, T>(k, ks, kbs, v, vs, vbs, t, heads, hd, tk, kp, vt, blockIdx.x * KB, blockIdx.y, blockIdx.z);
-  else if (blockIdx.z == 0) pack_pos<DP, T>(pos, ps, prow, hd, pfront, prows, pp, blockIdx.x - nkv, blockIdx.y);
+                                                   _Float16 *__restrict__ pp, Queries Q) {
+  const int nkv = tk / KB, np = pos ? prows / 32 : 0, x = blockIdx.x;
+  if (x < nkv) {
+    pack_kv<DP, T>(k, ks, kbs, v, vs, vbs, t, heads, hd, tk, kp, vt, x * KB, blockIdx.y, blockIdx.z);
+  } else if (x < nkv + np) {
+    if (blockIdx.z == 0) pack_pos<DP, T>(pos, ps, prow, hd, pfront, prows, pp, x - nkv, blockIdx.y);
+  } else if constexpr (std::is_same<T, float>::value) {
+    const int i = x - nkv - np, nq = (t + 31) / 32;
+    round_q<DP, T>(i < nq ? Q.q : Q.qv, Q.qs, t, hd, heads * hd, i < nq ? Q.q16 : Q.qv16, 32 * (i % nq), blockIdx.y, blockIdx.z);
+  }
 }
 
 // ---------------------------------------------------------------------------------- flash kernel
@@ -561,10 +613,10 @@ size_t split_bytes(int ns, int t, int heads, int hd, int batch) {
 
 template <int DP, typename T>
 void launch_pack(wh_ctx *ctx, const Pack &sp, const T *k, int ks, long kbs, const T *v, int vs, long vbs, const T *pos,
-                 int ps, int t, int heads, int hd, int batch, _Float16 *kp, _Float16 *vt, _Float16 *pp) {
-  const int gx = sp.tk / KB + (pos ? sp.prows / 32 : 0);
+                 int ps, int t, int heads, int hd, int batch, _Float16 *kp, _Float16 *vt, _Float16 *pp, const Queries &q) {
+  const int gx = sp.tk / KB + (pos ? sp.prows / 32 : 0) + (q.q ? (t + 31) / 32 * (q.qv ? 2 : 1) : 0);
   wh_launch(ctx, pack_kernel<DP, T>, dim3(gx, heads, batch), 256, 0, k, ks, kbs, v, vs, vbs, t, heads, hd, sp.tk, kp, vt,
-                                                                       pos, ps, 2 * t + 15, sp.pfront, sp.prows, pp);
+                                                                       pos, ps, 2 * t + 15, sp.pfront, sp.prows, pp, q);
 }
 
 template <bool REL>
@@ -625,9 +677,10 @@ int attention_t(wh_ctx *ctx, const T *qk, const T *v, const T *pos, int ps, void
   }
   const long bq = (long)t * qs, bv = (long)t * vs;
   const Pack sp = pack_shape(t, heads, hd, batch, pos != nullptr);
-  // Queries: f16 rows read by the flash kernel directly (f32 input: converted first, after the
+  // Queries: f16 rows read by the flash kernel directly (f32 input: rounded by the pack launch, after the
   // packed arrays in scratch).
-  const size_t qbytes = std::is_same<T, float>::value ? ((size_t)batch * t * qs * 2 + 255) / 256 * 256 : 0;
+  constexpr bool F32 = std::is_same<T, float>::value;
+  const size_t q1 = ((size_t)batch * t * ch * 2 + 255) / 256 * 256, qbytes = F32 ? q1 * (pos ? 2 : 1) : 0;
   a.nsplit = kv_splits(ctx, t, heads, hd, batch, pos != nullptr);
   uint8_t *ws = (uint8_t *)wh_scratch(ctx, sp.bytes() + qbytes + split_bytes(a.nsplit, t, heads, hd, batch));
   if (!ws) return WH_EOOM;
@@ -637,27 +690,25 @@ int attention_t(wh_ctx *ctx, const T *qk, const T *v, const T *pos, int ps, void
   }
   _Float16 *kp = (_Float16 *)ws, *vt = (_Float16 *)(ws + (sp.kv * 2 + 255) / 256 * 256);
   _Float16 *pp = (_Float16 *)(ws + 2 * ((sp.kv * 2 + 255) / 256 * 256));
+  Queries qr{};
+  if constexpr (F32) {
+    _Float16 *q16 = (_Float16 *)(ws + sp.bytes()), *qv16 = (_Float16 *)(ws + sp.bytes() + q1);
+    qr = {q, qv, q16, qv16, qs};
+    a.q = q16, a.qv = qv ? qv16 : nullptr, a.qs = ch;
+  } else {
+    a.q = q, a.qv = qv, a.qs = qs;
+  }
+  a.bq = (long)t * a.qs;
   {
     ProfScope prof(ctx, "attention_pack", 0.0,
-                   (sizeof(T) + 2.0) * batch * t * ch * 2 + (pos ? (sizeof(T) + 2.0) * (2 * t + 15) * ch : 0.0));
+                   (sizeof(T) + 2.0) * batch * t * ch * (F32 ? pos ? 4 : 3 : 2) + (pos ? (sizeof(T) + 2.0) * (2 * t + 15) * ch : 0.0));
     switch (sp.dp) {
-      case 32: launch_pack<32, T>(ctx, sp, k, qs, bq, vv, vs, bv, pos, ps, t, heads, hd, batch, kp, vt, pp); break;
-      case 64: launch_pack<64, T>(ctx, sp, k, qs, bq, vv, vs, bv, pos, ps, t, heads, hd, batch, kp, vt, pp); break;
-      default: launch_pack<128, T>(ctx, sp, k, qs, bq, vv, vs, bv, pos, ps, t, heads, hd, batch, kp, vt, pp); break;
+      case 32: launch_pack<32, T>(ctx, sp, k, qs, bq, vv, vs, bv, pos, ps, t, heads, hd, batch, kp, vt, pp, qr); break;
+      case 64: launch_pack<64, T>(ctx, sp, k, qs, bq, vv, vs, bv, pos, ps, t, heads, hd, batch, kp, vt, pp, qr); break;
+      default: launch_pack<128, T>(ctx, sp, k, qs, bq, vv, vs, bv, pos, ps, t, heads, hd, batch, kp, vt, pp, qr); break;
     }
     if (int rc = wh_launched(ctx, "attention pack")) return rc;
   }
-  if constexpr (std::is_same<T, float>::value) {
-    _Float16 *q16 = (_Float16 *)(ws + sp.bytes());
-    if (int rc = launch_to_half(ctx, qk, q16, (size_t)batch * t * qs)) return rc;
-    a.q = q16;
-    a.qv = qv ? q16 + 3 * ch : nullptr;
-  } else {
-    a.q = q;
-    a.qv = qv;
-  }
-  a.qs = qs;
-  a.bq = bq;
   a.kp = kp, a.vt = vt, a.pp = pp;
   a.tk = sp.tk, a.pfront = sp.pfront, a.prows = sp.prows;
   return pos ? launch_flash<true>(ctx, a, heads, batch, sp.dp) : launch_flash<false>(ctx, a, heads, batch, sp.dp);
@@ -723,8 +774,8 @@ int launch_attention(wh_ctx *ctx, const void *qk, const void *v, const void *pos
   if ((uintptr_t)qk % 16 || (v && (uintptr_t)v % 16) || (pos && (uintptr_t)pos % 16) || (uintptr_t)o % 16)
     return wh_fail(ctx, WH_EARG, "attention: buffers must be 16-byte aligned");
   const int ps = pos_stride > 0 ? pos_stride : heads * hd;
-  if (pos && ps < heads * hd)
-    return wh_fail(ctx, WH_EARG, "attention: position row stride %d below heads·hd %d", ps, heads * hd);
+  if (pos && (ps < heads * hd || ps % 4))
+    return wh_fail(ctx, WH_EARG, "attention: position row stride %d below heads·hd %d or no multiple of 4", ps, heads * hd);
   if (in16)
     return attention_t<_Float16>(ctx, (const _Float16 *)qk, (const _Float16 *)v, (const _Float16 *)pos, ps, o, t,
                                  heads, hd, valid_dev, valid, batch, out16);
