@@ -35,47 +35,61 @@
 #include "internal.h"
 #include "gemm_impl.h"
 
+// Shapes of about one 128×128 tile per CU or more: whole k, and the tile shape whose rounds over the CUs take
+// the least time.  Such a GEMM is bound by its last, partly filled round as much as by the tiles' own rate, so
+// no single tile is best over a range of rows (µs, Q8_0): 3000×4096×1024 is 51.0 as 96×128 tiles in two k
+// groups (3 rounds and an eighth of one) and 34.5 as 192×128 ones (one round, two workgroups per CU);
+// 3600×4096×1024 61.0 and, as 256×256 ones, 40.3; 2500×3840×1280 53.6 -> 37.0; 11616×1280×5120 198.6 -> 166.6.
+// Over 82 shapes of 1100 .. 11616 rows, 768 .. 5120 columns and k of 768 .. 5120 the choice below is within 1%
+// of the best of these tiles in the mean and 1.15 times as fast as one tile per range of tile counts.
+struct TileRounds {
+  GemmPlan plan;
+  int per_cu, per_cu_f16;  // workgroups that share a CU (LDS), with quantized and with F16 weights; 0: not taken
+  float t[3][2];  // a round with 1 .. per_cu workgroups per CU: t[·][0] + t[·][1] · k / 1024 µs, measured at k of 1024 .. 5120
+};
+constexpr TileRounds TILE_ROUNDS[] = {
+    {{96, 128, 1, 4, 3, 1, 0, 2}, 1, 1, {{7.0f, 6.5f}}},
+    {{96, 128, 1, 4, 3, 1}, 2, 1, {{6.0f, 8.0f}, {8.3f, 13.2f}}},
+    {{128, 128, 2, 4, 3, 1}, 2, 1, {{7.0f, 8.2f}, {7.5f, 18.2f}}},
+    {{128, 128, 2, 2, 2, 1}, 3, 2, {{7.8f, 9.0f}, {8.0f, 17.7f}, {8.7f, 26.8f}}},
+    {{192, 128, 2, 4, 2, 1}, 2, 2, {{8.5f, 11.5f}, {4.0f, 27.5f}}},
+    // (F16 weights have no dequantization that wavefronts of fewer columns would repeat)
+    {{256, 128, 2, 4, 3, 1}, 1, 0, {{9.2f, 16.6f}}},
+    {{256, 128, 4, 2, 2, 1}, 0, 1, {{9.2f, 16.6f}}},
+    {{192, 256, 2, 4, 2, 1}, 1, 1, {{6.7f, 25.8f}}},
+    {{256, 256, 2, 4, 2, 1}, 1, 1, {{8.4f, 31.6f}}},
+};
+
+GemmPlan least_rounds(int cus, int m, int cols, int k, bool f16) {
+  GemmPlan best = TILE_ROUNDS[0].plan;
+  float least = 0.0f;
+  for (const TileRounds &r : TILE_ROUNDS) {
+    const GemmPlan &p = r.plan;
+    const int per_cu = f16 ? r.per_cu_f16 : r.per_cu;
+    if (!per_cu || k % (64 * p.wk)) continue;
+    const long tiles = (long)((cols + p.bn - 1) / p.bn) * ((m + p.bm - 1) / p.bm), slots = (long)cus * per_cu;
+    auto round = [&](long wgs) { return r.t[(wgs - 1) / cus][0] + r.t[(wgs - 1) / cus][1] * (float)k / 1024.0f; };
+    const float t = (float)(tiles / slots) * round(slots) + (tiles % slots ? round(tiles % slots) : 0.0f);
+    if (least == 0.0f || t < least) least = t, best = p;
+  }
+  return best;
+}
+
 // Chosen per GEMM shape from measurements on MI355X (random operands, inside the encoder step, or
-// replayed back to back for m ≥ 1024): many output tiles → 256×256, 192×128 or 128×128 tiles; fewer
+// replayed back to back for m ≥ 1024): many output tiles → the tile shape with the cheapest rounds; fewer
 // → 64×64 tiles of 4 wavefronts, and when even those leave CUs idle, k split 2 or 4 ways.  Ring slots
 // of 64-wide k steps (a slot is refilled NS steps ahead, so NS − 1 steps hide the DMA's latency).
-GemmPlan gemm_plan_for(const wh_ctx *ctx, int m, int cols, int k) {
+GemmPlan gemm_plan_for(const wh_ctx *ctx, int m, int cols, int k, int type) {
+  const bool f16 = type == WH_F16;
   const int cus = ctx->cus > 0 ? ctx->cus : 256;
   const long t128 = (long)((cols + 127) / 128) * ((m + 127) / 128), t64 = (long)((cols + 63) / 64) * ((m + 63) / 64);
   GemmPlan p{64, 64, 2, 2, 3, 1};
-  const long t256 = (long)((cols + 255) / 256) * ((m + 255) / 256);
-  if (t128 >= 2L * cus && m >= 4096 && k >= 1024) {
-    // Two or more rounds of 128×128 tiles over many rows and a long k (batched windows, m ≈ 12000):
-    // wide outputs with at least two rounds of 256×256 tiles take those (8 wavefronts of 128×64, one
-    // workgroup per CU: the least a and W traffic per output — 12000×4096×1024 154 µs against 172 for
-    // 192×128 and 189 for 128×128); the others 192×128 tiles of 4 wavefronts, two workgroups per CU
-    // (12000×3072×1024 119 µs, 12000×1024×1024 44, 12000×1024×4096 152, against 131, 56 and 162 for
-    // 256×256 and 124, 47 and 162 for 128×128 tiles of 8).  (The batched position projection,
-    // 1515×24576×1024, streams its 27 MB of W from HBM in the step: 128×128 tiles, 2304 of them,
-    // run it in 128 µs there, 256×256 tiles in 189.)
-    if (cols >= 4096 && t256 >= 2L * cus) p = {256, 256, 2, 4, 2, 1};
-    else p = {192, 128, 2, 2, 2, 1};
-  } else if (t128 >= 4L * cus) p = {128, 128, 2, 4, 2, 1};
-  else if (t128 > cus && t128 <= 2L * cus && k < 4096)
-    // Between one and two 128×128 tiles per CU (a 1500-frame window's wide projections): 256×128
-    // tiles of 8 wavefronts with 64×64 wave tiles, one per CU, read each a fragment for twice the
-    // columns (measured in the Whisper encoder: 6.05 against 6.16 ms per call, fc1 1.28 against
-    // 1.35 ms, than 4-wave 128×128 tiles two per CU; at m = 12000 they are slower).
-    p = {256, 128, 4, 2, 2, 1};
-  else if (t128 > cus && (t128 <= 2L * cus || k >= 4096))
-    // More tiles than CUs with a long k (16 windows' FFN down projection): 4-wave workgroups in
-    // two slots, two per CU, take them in one round or fewer (measured in the encoder: 16 × 60 s
-    // FFN down 8.0 against 8.6 ms per call; the 16 windows' 1024 × 1024 projections stay with 8-wave
-    // workgroups, 3.13 against 3.22).
-    p = {128, 128, 2, 2, 2, 1};
-  else if (t128 * 4 >= 3L * cus)
-    // Three quarters of a tile per CU or more (the FFN's first projection at 750 frames): 96×128 tiles
-    // of one row of 4 wavefronts (96×32 each: every W fragment dequantized once per workgroup and fed
-    // to three MFMAs; 256 workgroups, one per CU) for k ≥ 1024 (60 s step 4.285 against 4.324 ms for
-    // 128×128 tiles of 2×4), in two k groups (15.7 against 16.0 µs in the step), else 128×128 tiles;
-    // fewer tiles (the qkv projection, 144) run faster as 64×64 tiles (4.96 against 4.98 ms per 60 s
-    // call; 96×128 tiles for it: 4.51 against 4.32).
-    p = k >= 1024 ? GemmPlan{96, 128, 1, 4, 3, 1, 0, 2} : GemmPlan{128, 128, 2, 4, 3, 1};
+  if (t128 * 4 >= 3L * cus || (t128 * 2 > cus && m >= 1024))
+    // Three quarters of a 128×128 tile per CU or more (the FFN's first projection at 750 frames: 96×128 tiles
+    // in two k groups, 256 of them), of many rows half a tile (1100×2048×1024 14.9 -> 12.0 µs, 2500×1024×1024
+    // 15.7 -> 13.8 as 96×128 tiles); with fewer rows 64×64 tiles stay ahead (the 750-frame qkv projection, 144
+    // of 128×128: the 60 s step 4.32 ms, 4.51 as 96×128 ones).
+    p = least_rounds(cus, m, cols, k, f16);
   else if (t128 * 4 <= cus && k % (4 * 64) == 0 && k / (4 * 64) >= 16)
     // Long k over few tiles (the FFN's down projection, 750 × 1024 × 4096): k split 4 ways over
     // 96×64 tiles of 2 wavefronts (96×32 per wavefront: each dequantized W fragment feeds three
@@ -85,7 +99,11 @@ GemmPlan gemm_plan_for(const wh_ctx *ctx, int m, int cols, int k) {
     // groups where they divide every split (14.3 against 15.0 µs in the step, the groups' sums in
     // LDS planes of their own).
     p = {96, 64, 1, 2, 2, 4, 0, k % (4 * 128) == 0 ? 2 : 1};
-  else if (t128 * 4 <= 2L * cus && k % 128 == 0 && k / (4 * 64) >= 16 &&
+  else if (f16 && t128 * 4 <= 2L * cus && k % (4 * 64) == 0 && k / (4 * 64) >= 16)
+    // F16 weights, whose ring of two k groups holds two slots only: k split (865×1472×4480, which cannot
+    // split, is 30.8 µs on 64×64 tiles below, 33.9 in the two groups).
+    p = {128, 128, 2, 2, 2, 4};
+  else if (!f16 && t128 * 4 <= 2L * cus && k % 128 == 0 && k / (4 * 64) >= 16 &&
            (long)((cols + 127) / 128) * ((m + 95) / 96) <= cus)
     // The same over up to half a 128×128 tile per CU (Whisper's fc2, 1500 × 1280 × 5120): the whole k in
     // two k groups over 96×128 tiles, 160 of them; no partial sums (four layers and their window 638 µs,
@@ -203,7 +221,7 @@ __global__ __launch_bounds__(256) void weight_tiles_kernel(const uint8_t *__rest
 
 // Scratch bytes for the split-k partial sums of an m-row GEMM (0 when it does not split).
 size_t split_bytes(const wh_ctx *ctx, const wh_linear *l, int m) {
-  const GemmPlan p = gemm_plan_for(ctx, m, l->cols, l->k);
+  const GemmPlan p = gemm_plan_for(ctx, m, l->cols, l->k, l->type);
   return p.split > 1 ? (size_t)p.split * m * l->cols * 4 : 0;
 }
 

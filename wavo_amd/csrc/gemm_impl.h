@@ -20,8 +20,8 @@ struct GemmPlan {
 // GemmPlan::pipe of the k-wavefront kernel (gemm_kw_kernel): bm × bn tiles of wk wavefronts.
 constexpr int PIPE_KW = 3;
 
-// The launch plan of an m × cols × k GEMM (gemm.hip).
-GemmPlan gemm_plan_for(const wh_ctx *ctx, int m, int cols, int k);
+// The launch plan of an m × cols × k GEMM with weights of a GGUF type (gemm.hip).
+GemmPlan gemm_plan_for(const wh_ctx *ctx, int m, int cols, int k, int type);
 
 namespace {
 
@@ -1309,9 +1309,11 @@ int kw_launch(wh_ctx *ctx, dim3 grid, const LdsArgs &a, const GemmPlan &p, bool 
 template <int WT>
 int launch_lds_t(wh_ctx *ctx, const _Float16 *a, const wh_linear *l, void *c, int m, int ldc, int epi, float alpha,
                  bool out16, float *part, int *splits, const HeadsOut *ho, int nho) {
-  GemmPlan p = gemm_plan_for(ctx, m, l->cols, l->k);
+  GemmPlan p = gemm_plan_for(ctx, m, l->cols, l->k, l->type);
   if (!l->wt) return wh_fail(ctx, WH_EARG, "gemm: a linear layer without weight tiles");
   if ((p.split > 1 && !part) || nho) p.split = 1;  // packed ranges are written by the tiles' own epilogue
+  for (int i = 0; i < nho; i++)  // packed ranges of whole 64-column tiles only
+    if (ho[i].col0 % p.bn || ho[i].cols % p.bn) p = {64, 64, 2, 2, 3, 1};
   if (splits) *splits = p.split;
   LdsArgs args{a, l->wt, l->bias, p.split > 1 ? (void *)part : c, m, l->rows, l->cols, l->k, l->dual, ldc, epi, alpha,
                {}, nho, nullptr, 0, 1};
@@ -1367,6 +1369,9 @@ int launch_lds_t(wh_ctx *ctx, const _Float16 *a, const wh_linear *l, void *c, in
     PLAN(128, 128, 2, 4, 2)
     PLAN(128, 128, 2, 2, 2)
     PLAN(256, 128, 4, 2, 2)
+    PLAN(256, 128, 2, 4, 3)
+    PLAN(192, 128, 2, 4, 2)
+    PLAN(192, 256, 2, 4, 2)
     PLAN(96, 64, 1, 2, 2)
     PLAN(192, 128, 2, 2, 2)
     PLAN(256, 256, 2, 4, 2)
