@@ -209,6 +209,26 @@ def test_gemm_k_wavefronts(gpu, wtype, plan):
         gpu.tune("gemm_plan", "")
 
 
+# Its a rows cross between the lanes of a wavefront through two LDS slots: shares of 3 to 21 k steps, even and
+# odd, so that each slot is written over and read again many times.
+@pytest.mark.parametrize("wtype", [wa.Q8_0, wa.Q4_0, wa.F16])
+@pytest.mark.parametrize("plan", ["32,32,1,1,2,1,3,8", "32,64,1,1,2,1,3,8", "64,64,1,1,2,1,3,4"])
+def test_gemm_k_wavefronts_reuse_their_slots(gpu, wtype, plan):
+    gpu.tune("gemm_plan", plan)
+    try:
+        for m, n, k in ((70, 96, 64 * 24), (70, 96, 64 * 81)):
+            w = np.random.default_rng(k).normal(0, 0.02, (n, k)).astype(np.float32)
+            raw, bias = ox.quantize(w, wtype), rnd(n, 2)
+            l, a = gpu.linear([(raw, wtype, k, n)], bias), rnd(m * k, 3).reshape(m, k)
+            cb = gpu.buffer(m * n)
+            gpu.gemm(gpu.upload(a), l, cb, m, wa.BIAS)
+            want = ox.gemm(a, ox.Linear(wtype, k, [(raw, n)], bias), m, wa.BIAS)
+            close(gpu.read(cb, (m, n)), want, tol=2e-5 * max(1.0, float(np.abs(want).max())),  # f32 sums, as above
+                  what=f"plan {plan} type {wtype} k {k}")
+    finally:
+        gpu.tune("gemm_plan", "")
+
+
 @pytest.mark.parametrize("plan", ["96,128,1,4,3,1,0,2", "96,64,1,2,2,4", "64,64,2,2,3,1"])
 def test_gemm_tile_orders_agree(gpu, plan):
     # The order in which XCDs take the tiles (groups of 1, 2, 3 and all row tiles, column by column

@@ -1150,6 +1150,13 @@ __global__ __launch_bounds__(64 * WK) void gemm_kw_kernel(LdsArgs P) {
 #pragma unroll
     for (int i = 0; i < TM; i++) f[i] = *(const half8 *)(mine + slot * A_ST + a_off[s] + 4096 * i);
   };
+  // Between a slot's writes and its reads, whose bytes other lanes wrote: the hardware runs a wavefront's LDS
+  // operations in order, this keeps the compiler from moving one over the other (no instruction of its own).
+  auto exchanged = [] {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  };
 
   constexpr int G8 = BN / 8;
   static_assert(NT % G8 == 0 && NT % BN == 0, "fixed column group per thread");
@@ -1180,6 +1187,7 @@ __global__ __launch_bounds__(64 * WK) void gemm_kw_kernel(LdsArgs P) {
   if (ns > 0) {
     write_a(ra[0], 0);
     if (2 < ns) load_a(ra[0], 2);
+    exchanged();
     read_a(af[0], 0, 0);
   }
   auto mma = [&](const half8 (&f)[TM], int set, auto s_c) {
@@ -1203,12 +1211,16 @@ __global__ __launch_bounds__(64 * WK) void gemm_kw_kernel(LdsArgs P) {
     __builtin_amdgcn_sched_barrier(0);
     read_a(af[1], S, 3);
     if (t + 1 < ns) {
+      exchanged();  // (step t − 1's reads of this slot come before)
       write_a(ra[1 - S], 1 - S);
       if (t + 3 < ns) load_a(ra[1 - S], t + 3);
     }
     mma(af[0], S, std::integral_constant<int, 2>{});
     __builtin_amdgcn_sched_barrier(0);
-    if (t + 1 < ns) read_a(af[0], 1 - S, 0);
+    if (t + 1 < ns) {
+      exchanged();
+      read_a(af[0], 1 - S, 0);
+    }
     mma(af[1], S, std::integral_constant<int, 3>{});
     if (t + 2 < ns) load_w(wq[S], ws[S], t + 2);
     __builtin_amdgcn_sched_barrier(0);
