@@ -93,6 +93,8 @@ void *wh_stream(wh_ctx *ctx);
  *                      (to time that kernel alone, as a model step runs it); "0" restores;
  *   "gemm_group"       "n": the GEMM's XCDs take tiles in groups of n row tiles, column by column inside a
  *                      group (0 = chosen per plan; the output is the same bit for bit);
+ *   "weight_tiles"     "0": layers that wh_linear_new creates from then on keep only their GGUF bytes; "1"
+ *                      restores (see there);
  *   "attn_split"       "n": attention splits its key range n ways (0 = chosen per shape);
  *   "position_cache"   "0": the Parakeet encoder recomputes its relative-position projection every call
  *                      instead of keeping it for the frame count its buffer holds (to time it); "1" restores;
@@ -149,7 +151,12 @@ typedef struct wh_tensor {
 
 /* Gpu::linear (src/gpu/mod.rs:758) and, with pad_k != 0, Gpu::conv (:766): the tensors stacked
  * along n, kept on the device in their GGUF bytes (Q8_0 34-byte / Q4_0 18-byte blocks as stored),
- * with the bias of the stacked rows (n_bias == 0: zeros).  A bias with `dual` more values than the
+ * with the bias of the stacked rows (n_bias == 0: zeros).  Q8_0, Q4_0 and F16 layers with k % 64 == 0
+ * are held a second time, in tiles that the GEMMs read (as many bytes again, rows rounded up to 32):
+ * the GEMV and the embedding read the GGUF bytes.  Where there is no memory for the tiles, or with
+ * wh_tune "weight_tiles" "0" (a layer that no GEMM reads needs none), the layer keeps its GGUF bytes
+ * alone and wh_gemm reads those, with the same results to the order of its f32 sums but at a small
+ * part of its speed.  (wh_model_load holds each weight once, in the form its readers take.)  A bias with `dual` more values than the
  * rows writes the first `dual` outputs again after the others with those biases (upload_linear,
  * :770-834).  k % 32 == 0 unless pad_k, which pads k to 32 with zero columns in F32 (exact, as the
  * GEMM rounds W to f16 either way). */

@@ -167,11 +167,10 @@ __global__ __launch_bounds__(256) void to_half_kernel(const float4 *__restrict__
   }
 }
 
-// The main kernel's conditions: 64-wide k steps over Q8_0 / Q4_0 / F16 rows, and an output whose
-// rows start on 16 bytes (its epilogue stores 8 columns at a time).
+// The main kernel's conditions: weight tiles (64-wide k steps over Q8_0 / Q4_0 / F16 weights), and an output
+// whose rows start on 16 bytes (its epilogue stores 8 columns at a time).
 bool lds_path(const wh_linear *l, const void *c, int ldc) {
-  return l->k % 64 == 0 && (l->type == WH_Q8_0 || l->type == WH_Q4_0 || l->type == WH_F16) && l->row_bytes % 4 == 0 &&
-         ldc % 8 == 0 && (uintptr_t)c % 16 == 0;
+  return l->wt && ldc % 8 == 0 && (uintptr_t)c % 16 == 0;
 }
 
 
@@ -267,6 +266,7 @@ int launch_t(wh_ctx *ctx, const void *a, const wh_linear *l, void *c, int m, int
 template <bool A16, bool OUT16>
 int launch_typed(wh_ctx *ctx, const void *a, const wh_linear *l, void *c, int m, int ldc, int epi, float alpha) {
   const bool aligned = l->k % 64 == 0;
+  if (!l->w) return wh_fail(ctx, WH_EARG, "gemm: only weight tiles are held, and the output is not 16-byte aligned");
   switch (l->type) {
     case WH_F32: return launch_t<WH_F32, true, A16, OUT16>(ctx, a, l, c, m, ldc, epi, alpha);
     case WH_F16: return launch_t<WH_F16, true, A16, OUT16>(ctx, a, l, c, m, ldc, epi, alpha);
@@ -293,10 +293,10 @@ size_t weight_tile_bytes(int type, int rows, int k) {
   return 0;
 }
 
-int launch_weight_tiles(wh_ctx *ctx, const wh_linear *l) {
+int launch_weight_tiles(wh_ctx *ctx, const wh_linear *l, const uint8_t *rows) {
   const size_t lanes = (size_t)((l->rows + 31) / 32) * (l->k / 64) * 64;
   const int blocks = (int)std::min<size_t>((lanes + 255) / 256, 16384);
-  auto go = [&](auto kernel) { wh_launch(ctx, kernel, blocks, 256, 0, (const uint8_t *)l->w, l->wt, l->rows, l->k / 64, l->row_bytes, lanes); };
+  auto go = [&](auto kernel) { wh_launch(ctx, kernel, blocks, 256, 0, rows, l->wt, l->rows, l->k / 64, l->row_bytes, lanes); };
   switch (l->type) {
     case WH_Q8_0: go(weight_tiles_kernel<WH_Q8_0>); break;
     case WH_Q4_0: go(weight_tiles_kernel<WH_Q4_0>); break;

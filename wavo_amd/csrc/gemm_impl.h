@@ -1322,7 +1322,6 @@ template <int WT>
 int launch_lds_t(wh_ctx *ctx, const _Float16 *a, const wh_linear *l, void *c, int m, int ldc, int epi, float alpha,
                  bool out16, float *part, int *splits, const HeadsOut *ho, int nho) {
   GemmPlan p = gemm_plan_for(ctx, m, l->cols, l->k, l->type);
-  if (!l->wt) return wh_fail(ctx, WH_EARG, "gemm: a linear layer without weight tiles");
   if ((p.split > 1 && !part) || nho) p.split = 1;  // packed ranges are written by the tiles' own epilogue
   for (int i = 0; i < nho; i++)  // packed ranges of whole 64-column tiles only
     if (ho[i].col0 % p.bn || ho[i].cols % p.bn) p = {64, 64, 2, 2, 3, 1};

@@ -106,6 +106,12 @@ struct wh_ctx {
   int pinned_slot = 0;
   size_t pinned_fill = 0;
   hipEvent_t upload_fence = nullptr;
+  // The rows of a LINEAR_TILES layer until its tiles are made (an event after that), for one layer after the
+  // other; held while a model loads.
+  uint8_t *tile_rows = nullptr;
+  size_t tile_rows_bytes = 0;
+  hipEvent_t tiles_made = nullptr;
+  int no_weight_tiles = 0;  // wh_tune "weight_tiles" 0
 };
 
 // A file whose mapping [base, base + size) a staged upload reads with pread instead of through the
@@ -122,9 +128,15 @@ int stage_upload(wh_ctx *ctx, void *dst, const void *src, size_t bytes, const St
 int stage_fence(wh_ctx *ctx);
 // Waits for every staged upload and reports their errors.
 int stage_wait(wh_ctx *ctx);
-// wh_linear_new with the weights read through `file` where they lie in its mapping.
+// What a linear layer's readers take: its rows as the GGUF stores them (GEMVs, the embedding, the transducer,
+// gemm_reg_kernel), its weight tiles (the other GEMMs), or either.
+enum LinearForm { LINEAR_BOTH, LINEAR_ROWS, LINEAR_TILES };
+// wh_linear_new with the weights read through `file` where they lie in its mapping, held in `form` only
+// (LINEAR_TILES where the layer has no tiles: rows).
 int linear_new(wh_ctx *ctx, const wh_tensor *ws, int count, const float *bias, int n_bias, int pad_k,
-               wh_linear **out, const StageFile *file);
+               wh_linear **out, const StageFile *file, LinearForm form);
+// Gives back the buffer that rows pass through on their way into tiles (LINEAR_TILES layers).
+void linear_stage_free(wh_ctx *ctx);
 
 // Looks up the device address of wh_gemm_noalloc's workspace on ctx's device (current), once per device.
 int gemm_noalloc_init(wh_ctx *ctx);
@@ -169,16 +181,18 @@ struct wh_linear {
   int k = 0;      // inner size (padded to 32 for a conv)
   int type = 0;   // WH_F32 / WH_F16 / WH_Q4_0 / WH_Q8_0
   size_t row_bytes = 0;
+  // Null where only GEMMs read the layer (LINEAR_TILES).
   uint8_t *w = nullptr;
   float *bias = nullptr;  // cols + dual values
-  // The same weights once more in the GEMM kernels' tiles (WTile), in the allocation of w; null for F32
-  // weights and k % 64 != 0, which those kernels do not take.
+  // The weights in the GEMM kernels' tiles (WTile).  Null for F32 weights and k % 64 != 0, which those kernels
+  // do not take, where no GEMM reads the layer (LINEAR_ROWS), and where the caller wants no second copy or
+  // there is no memory for it: gemm_reg_kernel then reads w.
   uint8_t *wt = nullptr;
 };
-// Bytes of a linear layer's weight tiles (0: none), and the kernel that makes them from l->w, on
+// Bytes of a linear layer's weight tiles (0: none), and the kernel that makes l->wt from the rows, on
 // ctx->stream.
 size_t weight_tile_bytes(int type, int rows, int k);
-int launch_weight_tiles(wh_ctx *ctx, const wh_linear *l);
+int launch_weight_tiles(wh_ctx *ctx, const wh_linear *l, const uint8_t *rows);
 
 // Sets ctx->error and returns code.
 int wh_fail(wh_ctx *ctx, int code, const char *fmt, ...);

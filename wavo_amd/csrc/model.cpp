@@ -322,9 +322,10 @@ class Loader {
   }
 
   // conformer::linear / transformer::stacked: the weights `names[i].weight` stacked along n with
-  // their biases (index `zero` has none: Whisper's k); `extra` appended after (dual outputs).
+  // their biases (index `zero` has none: Whisper's k); `extra` appended after (dual outputs).  Each layer is
+  // held once, in the form its readers take: tiles where GEMMs into the model's own buffers read it.
   wh_linear *linear(const std::vector<std::string> &names, bool bias, int zero = -1,
-                    const std::vector<float> &override_bias = {}, int pad_k = 0) {
+                    const std::vector<float> &override_bias = {}, int pad_k = 0, LinearForm form = LINEAR_TILES) {
     if (!err.empty()) return nullptr;
     std::vector<wh_tensor> ws;
     std::vector<float> b;
@@ -347,7 +348,7 @@ class Loader {
     wh_linear *l = nullptr;
     const StageFile file = g_.file();
     if (linear_new(ctx_, ws.data(), (int)ws.size(), bb.empty() ? nullptr : bb.data(), (int)bb.size(), pad_k, &l,
-                   &file)) {
+                   &file, form)) {
       fail(names[0] + ": " + ctx_->error);
       return nullptr;
     }
@@ -359,6 +360,14 @@ class Loader {
   // its rows permuted into groups of 8, [x 4j .. 4j+3 | gates 4j .. 4j+3] for j = 0 .. ch/4 − 1, so
   // that a GEMM epilogue holds every channel's x and gate in one lane (EPI_GLU); *groups says whether
   // it did (ch % 4 == 0), else the rows stay as stored.  Whole rows move: the products are unchanged.
+  // A layer that only GEMVs, the embedding or the transducer read.
+  wh_linear *rows(const std::vector<std::string> &names, bool bias, int zero = -1) {
+    return linear(names, bias, zero, {}, 0, LINEAR_ROWS);
+  }
+
+  // A layer whose GEMM writes into the caller's buffer, which may lie off the main kernel's 16-byte alignment.
+  wh_linear *head(const std::vector<std::string> &names) { return linear(names, true, -1, {}, 0, LINEAR_BOTH); }
+
   wh_linear *glu_groups(const std::string &name, bool bias, bool *groups) {
     *groups = false;
     if (!err.empty()) return nullptr;
@@ -378,7 +387,7 @@ class Loader {
     }
     wh_tensor w{host.data(), t->type, k, rows};
     wh_linear *l = nullptr;
-    if (linear_new(ctx_, &w, 1, b.empty() ? nullptr : b.data(), (int)b.size(), 0, &l, nullptr)) {
+    if (linear_new(ctx_, &w, 1, b.empty() ? nullptr : b.data(), (int)b.size(), 0, &l, nullptr, LINEAR_TILES)) {
       fail(name + ": " + ctx_->error);
       return nullptr;
     }
@@ -415,7 +424,7 @@ class Loader {
     }
     wh_tensor w{host.data(), type, k, rows};
     wh_linear *l = nullptr;
-    if (linear_new(ctx_, &w, 1, bias.data(), (int)bias.size(), 0, &l, nullptr)) {
+    if (linear_new(ctx_, &w, 1, bias.data(), (int)bias.size(), 0, &l, nullptr, LINEAR_ROWS)) {
       fail(names[0] + ": " + ctx_->error);
       return nullptr;
     }
@@ -695,7 +704,7 @@ bool load_parakeet(const Gguf &g, Loader &L, wh_model *m, std::string &err) {
   m->conv3 = L.linear({"enc.pre_encode.conv.3"}, true);
   m->conv6 = L.linear({"enc.pre_encode.conv.6"}, true);
   m->pre_out = L.linear({"enc.pre_encode.out"}, true);
-  m->joint_enc = L.linear({"joint.enc"}, true);
+  m->joint_enc = L.head({"joint.enc"});
   m->blocks.resize(m->layers);
   for (int i = 0; i < m->layers && L.err.empty(); i++) load_block(L, m, i, m->blocks[i]);
   {
@@ -732,8 +741,8 @@ bool load_parakeet(const Gguf &g, Loader &L, wh_model *m, std::string &err) {
         std::string p = "pred.lstm." + std::to_string(l);
         m->tdt_lstm.push_back(L.joined({p + ".Wx", p + ".Wh"}, m->lstm_b[l]));
       }
-      m->tdt_pred = L.linear({"joint.pred"}, true);
-      m->tdt_out = L.linear({"joint.out"}, true);
+      m->tdt_pred = L.rows({"joint.pred"}, true);
+      m->tdt_out = L.rows({"joint.out"}, true);
       m->tdt_embed = L.upload(m->embed_h.w);
     }
   }
@@ -754,7 +763,7 @@ bool load_gigaam(const Gguf &g, Loader &L, wh_model *m, std::string &err) {
   m->conv0 = L.linear({"enc.pre_encode.conv.0"}, true);
   m->conv2 = L.linear({"enc.pre_encode.conv.2"}, true);
   bool rnnt = g.string("stt.gigaam.head_kind") == "rnnt";
-  m->head = L.linear({rnnt ? "joint.enc" : "head.ctc"}, true);
+  m->head = L.head({rnnt ? "joint.enc" : "head.ctc"});
   const Tensor *ht = g.tensor(rnnt ? "joint.enc.weight" : "head.ctc.weight");
   m->outputs = ht ? (int)ht->dims.back() : 0;
   m->blank = (int)g.integer("tokenizer.ggml.blank_token_id", -1);
@@ -806,15 +815,15 @@ bool load_whisper(const Gguf &g, Loader &L, wh_model *m, std::string &err) {
     std::string p = "dec.blocks." + std::to_string(i) + ".";
     DLayer &l = m->dl[i];
     l.norm_self = L.norm(p + "norm_self", d, true);
-    l.qkv = L.linear({p + "self_attn.q", p + "self_attn.k", p + "self_attn.v"}, true, 1);
-    l.self_out = L.linear({p + "self_attn.out"}, true);
+    l.qkv = L.rows({p + "self_attn.q", p + "self_attn.k", p + "self_attn.v"}, true, 1);
+    l.self_out = L.rows({p + "self_attn.out"}, true);
     l.norm_cross = L.norm(p + "norm_cross", d, true);
-    l.cross_q = L.linear({p + "cross_attn.q"}, true);
+    l.cross_q = L.rows({p + "cross_attn.q"}, true);
     l.cross_kv = L.linear({p + "cross_attn.k", p + "cross_attn.v"}, true, 0);
-    l.cross_out = L.linear({p + "cross_attn.out"}, true);
+    l.cross_out = L.rows({p + "cross_attn.out"}, true);
     l.norm_ffn = L.norm(p + "norm_ffn", d, true);
-    l.fc1 = L.linear({p + "ffn.fc1"}, true);
-    l.fc2 = L.linear({p + "ffn.fc2"}, true);
+    l.fc1 = L.rows({p + "ffn.fc1"}, true);
+    l.fc2 = L.rows({p + "ffn.fc2"}, true);
   }
   m->dec_norm = L.norm("dec.final_norm", d, true);
   m->eot = (int)g.integer("tokenizer.ggml.eos_token_id", -1);
@@ -830,7 +839,7 @@ bool load_whisper(const Gguf &g, Loader &L, wh_model *m, std::string &err) {
     for (int id : m->begin_suppress) ok = ok && id >= 0 && id < m->vocab;
     if (!ok) return err = "special token ids out of the vocabulary", false;
   }
-  m->token_embd = L.linear({"dec.token_embd"}, false);
+  m->token_embd = L.rows({"dec.token_embd"}, false);
   m->dec_pos = L.upload(L.f32s("dec.pos_emb.weight", (size_t)d * m->context));
   return L.err.empty();
 }
@@ -1824,6 +1833,7 @@ int wh_model_load(wh_ctx *ctx, const char *path, wh_model **out) {
   m->linears = L.linears;
   // Every staged upload done (and its errors seen) before the model is handed out.
   if (ok && L.err.empty() && (stage_fence(ctx) || stage_wait(ctx))) L.fail(ctx->error);
+  linear_stage_free(ctx);
   if (!ok || !L.err.empty()) {
     std::string msg = err.empty() ? L.err : err;
     wh_model_free(m.release());

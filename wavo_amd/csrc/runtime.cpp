@@ -148,6 +148,7 @@ void wh_close(wh_ctx *ctx) {
   if (!ctx) return;
   (void)hipSetDevice(ctx->device);
   (void)hipStreamSynchronize(ctx->stream);
+  linear_stage_free(ctx);
   if (ctx->upload) {
     (void)hipStreamSynchronize(ctx->upload);
     for (int i = 0; i < wh_ctx::STAGE_SLOTS; i++) {
@@ -397,6 +398,8 @@ int wh_tune(wh_ctx *ctx, const char *key, const char *value) {
     ctx->gemm_kernel_only = atoi(v) != 0;
   } else if (!strcmp(key, "position_cache")) {
     ctx->no_position_cache = atoi(v) == 0;
+  } else if (!strcmp(key, "weight_tiles")) {
+    ctx->no_weight_tiles = *v && atoi(v) == 0;
   } else if (!strcmp(key, "gemm_group")) {
     ctx->gemm_group = std::max(0, atoi(v));
   } else if (!strcmp(key, "attn_split")) {
@@ -557,13 +560,40 @@ int wh_profile_read(wh_ctx *ctx, char *out, size_t len) {
 
 int wh_linear_new(wh_ctx *ctx, const wh_tensor *ws, int count, const float *bias, int n_bias,
                   int pad_k, wh_linear **out) {
-  return linear_new(ctx, ws, count, bias, n_bias, pad_k, out, nullptr);
+  const LinearForm form = ctx && ctx->no_weight_tiles ? LINEAR_ROWS : LINEAR_BOTH;
+  return linear_new(ctx, ws, count, bias, n_bias, pad_k, out, nullptr, form);
 }
 
 }  // extern "C"
 
+// The buffer that a LINEAR_TILES layer's rows pass through, at least `bytes`; the uploads queued from here on
+// wait until the last layer's tiles are made from it.
+static hipError_t tile_rows_reserve(wh_ctx *ctx, size_t bytes) {
+  hipError_t e = hipSuccess;
+  if (stage_init(ctx)) return hipErrorOutOfMemory;
+  if (!ctx->tiles_made) e = hipEventCreateWithFlags(&ctx->tiles_made, hipEventDisableTiming);
+  if (e == hipSuccess && bytes > ctx->tile_rows_bytes) {
+    (void)hipStreamSynchronize(ctx->upload), (void)hipStreamSynchronize(ctx->stream);
+    if (ctx->tile_rows) (void)hipFree(ctx->tile_rows);
+    ctx->tile_rows = nullptr, ctx->tile_rows_bytes = 0;
+    e = hipMalloc(&ctx->tile_rows, bytes);
+    if (e != hipSuccess) ctx->tile_rows = nullptr;
+    else ctx->tile_rows_bytes = bytes;
+  }
+  if (e == hipSuccess) e = hipStreamWaitEvent(ctx->upload, ctx->tiles_made, 0);
+  return e;
+}
+
+void linear_stage_free(wh_ctx *ctx) {
+  if (ctx->upload) (void)hipStreamSynchronize(ctx->upload);
+  if (ctx->tile_rows) (void)hipStreamSynchronize(ctx->stream), (void)hipFree(ctx->tile_rows);
+  ctx->tile_rows = nullptr, ctx->tile_rows_bytes = 0;
+  if (ctx->tiles_made) (void)hipEventDestroy(ctx->tiles_made);
+  ctx->tiles_made = nullptr;
+}
+
 int linear_new(wh_ctx *ctx, const wh_tensor *ws, int count, const float *bias, int n_bias, int pad_k,
-               wh_linear **out, const StageFile *file) {
+               wh_linear **out, const StageFile *file, LinearForm form) {
   if (!ctx || !ws || count <= 0 || !out || n_bias < 0) return wh_fail(ctx, WH_EARG, "wh_linear_new: bad arguments");
   if (ctx->recording) return wh_fail(ctx, WH_EARG, "wh_linear_new: weights cannot be created while recording");
   *out = nullptr;
@@ -624,13 +654,22 @@ int linear_new(wh_ctx *ctx, const wh_tensor *ws, int count, const float *bias, i
   l->row_bytes = wh_type_bytes(dtype, (size_t)kp);
   (void)hipSetDevice(ctx->device);
   size_t wbytes = l->row_bytes * rows;
-  // 256 bytes of slack: the GEMM's loaders read whole dwords of the last row.
-  // Then, on a 256-byte boundary, the weight tiles: as many bytes again, made once, so that the GEMMs load
-  // W in whole lines (see gemm.hip).
-  const size_t tiles = weight_tile_bytes(dtype, rows, kp), at_tiles = (wbytes + 256 + 255) / 256 * 256;
-  hipError_t e = hipMalloc(&l->w, tiles ? at_tiles + tiles : wbytes + 256);
-  if (e == hipSuccess && tiles) l->wt = l->w + at_tiles;
+  // Rows and weight tiles (see gemm.hip) each in an allocation of their own, the rows with 256 bytes of slack:
+  // the GEMMs' and GEMVs' loaders read whole dwords of the last row.  A layer held as tiles only passes its rows
+  // through the context's buffer.  For a caller's layer the tiles are a second copy: without memory for them it
+  // keeps its rows alone.
+  const size_t tiles = form == LINEAR_ROWS ? 0 : weight_tile_bytes(dtype, rows, kp);
+  const bool passing = tiles && form == LINEAR_TILES;
+  hipError_t e = hipSuccess;
+  if (!passing) e = hipMalloc(&l->w, wbytes + 256);
   if (e == hipSuccess) e = hipMalloc(&l->bias, sizeof(float) * (size_t)(n > cols + dual ? n : cols + dual));
+  if (e == hipSuccess && tiles) {
+    e = hipMalloc(&l->wt, tiles);
+    if (e != hipSuccess) l->wt = nullptr;
+    if (e == hipErrorOutOfMemory && !passing) (void)hipGetLastError(), e = hipSuccess;
+  }
+  if (e == hipSuccess && passing) e = tile_rows_reserve(ctx, wbytes + 256);
+  uint8_t *const w = passing ? ctx->tile_rows : l->w;
   if (e != hipSuccess) {
     (void)hipGetLastError();
     int rc = wh_fail(ctx, e == hipErrorOutOfMemory ? WH_EOOM : WH_EGPU, "weights: %s", hipGetErrorString(e));
@@ -646,19 +685,21 @@ int linear_new(wh_ctx *ctx, const wh_tensor *ws, int count, const float *bias, i
   static const uint8_t zeros[256] = {};
   int rc = WH_OK;
   if (!host.empty()) {
-    rc = stage_upload(ctx, l->w, host.data(), wbytes);
+    rc = stage_upload(ctx, w, host.data(), wbytes);
   } else {
     size_t at = 0;
     for (int i = 0; i < count && rc == WH_OK; i++) {
       size_t b = l->row_bytes * ws[i].rows;
-      rc = stage_upload(ctx, l->w + at, ws[i].data, b, file);
+      rc = stage_upload(ctx, w + at, ws[i].data, b, file);
       at += b;
     }
   }
-  if (rc == WH_OK) rc = stage_upload(ctx, l->w + wbytes, zeros, sizeof zeros);
+  if (rc == WH_OK) rc = stage_upload(ctx, w + wbytes, zeros, sizeof zeros);
   if (rc == WH_OK) rc = stage_upload(ctx, l->bias, pb.data(), sizeof(float) * pb.size());
   if (rc == WH_OK) rc = stage_fence(ctx);
-  if (rc == WH_OK && l->wt) rc = launch_weight_tiles(ctx, l);
+  if (rc == WH_OK && l->wt) rc = launch_weight_tiles(ctx, l, w);
+  if (rc == WH_OK && passing && hipEventRecord(ctx->tiles_made, ctx->stream) != hipSuccess)
+    rc = wh_fail(ctx, WH_EGPU, "weight tiles: %s", hipGetErrorString(hipGetLastError()));
   if (rc != WH_OK) {
     (void)stage_wait(ctx);
     wh_linear_free(ctx, l);
@@ -679,6 +720,7 @@ void wh_linear_free(wh_ctx *ctx, wh_linear *l) {
   if (ctx) (void)hipSetDevice(ctx->device);
   if (ctx && ctx->upload) (void)hipStreamSynchronize(ctx->upload);  // no copy into it still queued
   if (l->w) (void)hipFree(l->w);
+  if (l->wt) (void)hipFree(l->wt);
   if (l->bias) (void)hipFree(l->bias);
   delete l;
 }
