@@ -1,0 +1,55 @@
+"""The GEMM's launch plan over the ranges of its rules: the kernel that a call takes, by its profiled name, and
+sampled rows of its output against the oracle, at the tolerance of the sweep (f32 sums in another order)."""
+
+import functools
+
+import numpy as np
+import pytest
+
+import oracle as ox
+import wavo_amd as wa
+from wavo_amd import gguf
+
+pytestmark = pytest.mark.gpu
+
+KW32, KW3264, KW64 = "32x32_w1x1_n2_p3_k8", "32x64_w1x1_n2_p3_k8", "64x64_w1x1_n2_p3_k4"
+NAMES = {wa.Q8_0: "q8_0", wa.Q4_0: "q4_0", wa.F16: "f16"}
+
+
+@functools.lru_cache(maxsize=2)
+def weights(n, k, wtype):
+    w = np.random.default_rng(n * 7 + k).standard_normal(n * k, dtype=np.float32) * np.float32(0.02)
+    return gguf.encode(w, wtype), np.random.default_rng(n).standard_normal(n, dtype=np.float32)
+
+
+def check(gpu, m, n, k, wtype, plan, out16=False):
+    raw, bias = weights(n, k, wtype)
+    l = gpu.linear([(raw, wtype, k, n)], bias)
+    a = np.random.default_rng(m + k).standard_normal((m, k), dtype=np.float32)
+    ah = gpu.upload(a.astype(np.float16))
+    cb = gpu.buffer(m * l.width)
+    gpu.profile(1)
+    try:
+        gpu.gemm_h(ah, l, cb, m, wa.BIAS, 0.0, out16=out16)
+        names = [x["kernel"].split(" ")[0] for x in gpu.profile_read()]
+    finally:
+        gpu.profile(0)
+    assert names[0] == f"gemm_{NAMES[wtype]}_{plan}", f"{m}x{n}x{k} {NAMES[wtype]}: {names}"
+    rng = np.random.default_rng(m)
+    rows = np.unique(np.concatenate([[0, m - 1], rng.choice(m, min(m, 24), replace=False)]))
+    dtype = np.float16 if out16 else np.float32
+    size = np.dtype(dtype).itemsize
+    got = np.stack([gpu.read(cb, (l.width,), dtype, offset_bytes=size * int(r) * l.width) for r in rows])[:, :n].astype(np.float32)
+    want = ox.gemm(a[rows], ox.Linear(wtype, k, [(raw, n)], bias), len(rows), ox.BIAS)
+    top = max(1.0, float(np.abs(want).max()))
+    tol = (2e-5 + (2.0 ** -11 if out16 else 0.0)) * top  # (f16 outputs: rounded once)
+    assert np.abs(got - want).max() <= tol, f"{m}x{n}x{k} {NAMES[wtype]} {plan}"
+
+
+# Wavefronts that split k: not over one k step (of 64), on 32x64 tiles not over two, from there on yes.
+@pytest.mark.parametrize("m,n,k,wtype,plan", [
+    (28, 832, 64, wa.Q8_0, "64x64_w2x2_n3"), (3, 4800, 64, wa.F16, "64x64_w2x2_n3"), (260, 1408, 64, wa.Q4_0, "64x64_w2x2_n3"),
+    (2020, 160, 128, wa.Q4_0, "64x64_w2x2_n4_k2"), (44, 576, 128, wa.Q4_0, KW32), (11, 128, 128, wa.F16, KW32),
+    (1133, 288, 192, wa.Q8_0, KW3264), (465, 800, 512, wa.Q4_0, KW3264), (60, 1024, 4096, wa.F16, KW32)])
+def test_k_wavefronts_need_k_to_split(gpu, m, n, k, wtype, plan):
+    check(gpu, m, n, k, wtype, plan)

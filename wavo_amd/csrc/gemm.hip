@@ -128,7 +128,9 @@ GemmPlan gemm_plan_for(const wh_ctx *ctx, int m, int cols, int k, int type) {
   // (one workgroup per CU), whose chain of steps is then the shortest.  µs per encoder call with that one
   // layer on the LDS-DMA kernel and here: 60 Parakeet frames 2 289 against 2 073 for the 1024 × 1024
   // projections (32×32 tiles), 2 298 for 4096 × 1024 (32×64), 2 807 for all of them; 275 GigaAM frames
-  // 1 790 against 1 682 for the 768 × 768 ones, 1 854 for 768 × 3072.  With 64×64 tiles the LDS-DMA
+  // 1 790 against 1 682 for the 768 × 768 ones, 1 854 for 768 × 3072.  Not over one or two steps of k, whose sums
+  // cost more than the split saves (recorded, one after the other: 260×1408×64 3.9 on the LDS-DMA kernel, 4.3
+  // here, 2020×160×128 4.2 and 4.4 on 32×64 tiles, but 103×96×128 4.2 and 3.7).  With 64×64 tiles the LDS-DMA
   // kernel's two k groups are the faster ones while the tiles run at once (750 frames' 1024 × 1024: 3 584
   // against 3 626; 275 frames' 3072 × 1024: 2 846 against 2 886), this kernel for one to two tiles per CU
   // of few rows (750 frames' 2048 × 1024: 3 630 against 3 605; 500 frames' 3072 × 1024: 3 153 against
@@ -136,8 +138,8 @@ GemmPlan gemm_plan_for(const wh_ctx *ctx, int m, int cols, int k, int type) {
   {
     const long t32 = (long)((cols + 31) / 32) * ((m + 31) / 32), t3264 = (long)((cols + 63) / 64) * ((m + 31) / 32);
     if ((size_t)m * k < ((size_t)1 << 30)) {  // 32-bit byte offsets into a
-      if (t32 <= cus) p = {32, 32, 1, 1, 2, 1, PIPE_KW, 8};
-      else if (t3264 <= cus) p = {32, 64, 1, 1, 2, 1, PIPE_KW, 8};
+      if (t32 <= cus && k >= 128) p = {32, 32, 1, 1, 2, 1, PIPE_KW, 8};
+      else if (t32 > cus && t3264 <= cus && k >= 192) p = {32, 64, 1, 1, 2, 1, PIPE_KW, 8};
       else if (m < 1024 && k <= 2048 && t64 > cus && t64 <= 2L * cus) p = {64, 64, 1, 1, 2, 1, PIPE_KW, 4};
     }
   }
