@@ -83,6 +83,7 @@ GemmPlan gemm_plan_for(const wh_ctx *ctx, int m, int cols, int k, int type) {
   const bool f16 = type == WH_F16;
   const int cus = ctx->cus > 0 ? ctx->cus : 256;
   const long t128 = (long)((cols + 127) / 128) * ((m + 127) / 128), t64 = (long)((cols + 63) / 64) * ((m + 63) / 64);
+  const long t9664 = (long)((cols + 63) / 64) * ((m + 95) / 96);
   GemmPlan p{64, 64, 2, 2, 3, 1};
   if (t128 * 4 >= 3L * cus || (t128 * 2 > cus && m >= 1024))
     // Three quarters of a 128×128 tile per CU or more (the FFN's first projection at 750 frames: 96×128 tiles
@@ -119,10 +120,12 @@ GemmPlan gemm_plan_for(const wh_ctx *ctx, int m, int cols, int k, int type) {
     // 1024 × 1024 projections 9.5 against 10.0 µs in the step; deeper rings alone are slower there:
     // 10.8 for 5 slots, 11.4 for 8).
     if (p.split == 1 && k % 128 == 0) p = {64, 64, 2, 2, 4, 1, 0, 2};
-  } else if (t64 < 2L * cus)
+  } else if (t64 < 2L * cus && !(f16 && (k % 128 || (t9664 > cus && k <= 1024))))
     // One to two 64×64 tiles per CU (the 750-frame pointwise projection, 750 × 2048 × 1024): 96×64
     // tiles of one row of 2 wavefronts in two k groups, one workgroup per CU (11.7 against 12.7 µs
-    // in the step for 64×64 tiles; 12.2 with 4 slots).
+    // in the step for 64×64 tiles; 12.2 with 4 slots).  F16 weights stay on 64×64 tiles over an odd number of
+    // steps (918×1472×1984 15.7 against 20.4) and over more than a 96×64 tile per CU of a short k
+    // (937×1728×1024 11.6 against 12.9; 623×2688×1536 15.4 and 16.0, 571×3520×1920 20.7 and 19.5).
     p = {96, 64, 1, 2, 2, 1, 0, 2};
   // Few tiles: wavefronts that split k (gemm_kw_kernel), the smallest of its tiles that still run at once
   // (one workgroup per CU), whose chain of steps is then the shortest.  µs per encoder call with that one
@@ -132,15 +135,18 @@ GemmPlan gemm_plan_for(const wh_ctx *ctx, int m, int cols, int k, int type) {
   // cost more than the split saves (recorded, one after the other: 260×1408×64 3.9 on the LDS-DMA kernel, 4.3
   // here, 2020×160×128 4.2 and 4.4 on 32×64 tiles, but 103×96×128 4.2 and 3.7).  With 64×64 tiles the LDS-DMA
   // kernel's two k groups are the faster ones while the tiles run at once (750 frames' 1024 × 1024: 3 584
-  // against 3 626; 275 frames' 3072 × 1024: 2 846 against 2 886), this kernel for one to two tiles per CU
-  // of few rows (750 frames' 2048 × 1024: 3 630 against 3 605; 500 frames' 3072 × 1024: 3 153 against
-  // 3 105; Whisper's 1500 rows and tiles past two per CU stay above).
+  // against 3 626; 275 frames' 3072 × 1024: 2 846 against 2 886), and so are its 96×64 ones above
+  // (750×2048×1024 10.7 there, 12.5 here; 458×2752×1920 Q4_0 13.3 and 16.0); this kernel for one to two tiles per
+  // CU of few rows whose 96×64 tiles are too many or walk an odd number of steps (500×3072×1024 12.4 and 12.2,
+  // 392×3520×1728 22.5 and 16.4), with Q8_0 and Q4_0: with F16 weights it holds over 256 registers, one
+  // workgroup per CU (595×2368×896 11.7 on 96×64 tiles, 10.4 on 64×64 ones, 14.5 here).
   {
     const long t32 = (long)((cols + 31) / 32) * ((m + 31) / 32), t3264 = (long)((cols + 63) / 64) * ((m + 31) / 32);
     if ((size_t)m * k < ((size_t)1 << 30)) {  // 32-bit byte offsets into a
       if (t32 <= cus && k >= 128) p = {32, 32, 1, 1, 2, 1, PIPE_KW, 8};
       else if (t32 > cus && t3264 <= cus && k >= 192) p = {32, 64, 1, 1, 2, 1, PIPE_KW, 8};
-      else if (m < 1024 && k <= 2048 && t64 > cus && t64 <= 2L * cus) p = {64, 64, 1, 1, 2, 1, PIPE_KW, 4};
+      else if (!f16 && m < 1024 && k <= 2048 && t64 > cus && t64 <= 2L * cus && (t9664 > cus || k % 128))
+        p = {64, 64, 1, 1, 2, 1, PIPE_KW, 4};
     }
   }
   if (ctx->gemm_plan[0]) {  // tuning override (wh_tune "gemm_plan"): bm, bn, wm, wn, stages, split, pipeline, kgroups
