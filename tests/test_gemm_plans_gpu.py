@@ -65,3 +65,15 @@ def test_k_wavefronts_need_k_to_split(gpu, m, n, k, wtype, plan):
 @pytest.mark.parametrize("out16", [False, True])
 def test_one_to_two_tiles_per_cu(gpu, m, n, k, wtype, plan, out16):
     check(gpu, m, n, k, wtype, plan, out16)
+
+
+# A long k: split over few tiles, whole in two k groups from there on, on the widest of the 64x64, 96x64 and 96x128
+# tiles that still gives every CU one.  k of pairs of steps that no split into four divides (4224, 4992) as well.
+@pytest.mark.parametrize("m,n,k,wtype,plan", [
+    (750, 1024, 4096, wa.Q8_0, "96x64_w1x2_n2_s4_k2"), (166, 2752, 4224, wa.Q8_0, "64x64_w2x2_n4_k2"),
+    (400, 1408, 4992, wa.Q4_0, "64x64_w2x2_n4_k2"), (1024, 1024, 4224, wa.F16, "64x64_w2x2_n4_k2"),
+    (549, 1664, 4608, wa.F16, "64x64_w2x2_n4_k2"), (750, 1792, 4096, wa.Q4_0, "96x64_w1x2_n2_k2"), (670, 1664, 4224, wa.Q4_0, "96x64_w1x2_n2_k2"),
+    (300, 4288, 4224, wa.Q4_0, "96x128_w1x4_n3_k2"), (1500, 1280, 5120, wa.Q8_0, "96x128_w1x4_n3_k2"),
+    (757, 1792, 4096, wa.F16, "128x128_w2x2_n2_s4")])
+def test_long_k(gpu, m, n, k, wtype, plan):
+    check(gpu, m, n, k, wtype, plan)

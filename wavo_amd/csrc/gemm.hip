@@ -100,26 +100,25 @@ GemmPlan gemm_plan_for(const wh_ctx *ctx, int m, int cols, int k, int type) {
     // groups where they divide every split (14.3 against 15.0 µs in the step, the groups' sums in
     // LDS planes of their own).
     p = {96, 64, 1, 2, 2, 4, 0, k % (4 * 128) == 0 ? 2 : 1};
-  else if (f16 && t128 * 4 <= 2L * cus && k % (4 * 64) == 0 && k / (4 * 64) >= 16)
+  else if (f16 && t64 > cus && t128 * 4 <= 2L * cus && k % (4 * 64) == 0 && k / (4 * 64) >= 16)
     // F16 weights, whose ring of two k groups holds two slots only: k split (865×1472×4480, which cannot
     // split, is 30.8 µs on 64×64 tiles below, 33.9 in the two groups).
     p = {128, 128, 2, 2, 2, 4};
-  else if (!f16 && t128 * 4 <= 2L * cus && k % 128 == 0 && k / (4 * 64) >= 16 &&
-           (long)((cols + 127) / 128) * ((m + 95) / 96) <= cus)
+  else if (!f16 && t9664 > cus && t128 * 4 <= 2L * cus && k % 128 == 0 && k / (4 * 64) >= 16)
     // The same over up to half a 128×128 tile per CU (Whisper's fc2, 1500 × 1280 × 5120): the whole k in
     // two k groups over 96×128 tiles, 160 of them; no partial sums (four layers and their window 638 µs,
-    // against 645 for 128×128 tiles with k split 4 ways, 640 for 96×64 tiles, 676 split 2 ways).
+    // against 645 for 128×128 tiles with k split 4 ways, 640 for 96×64 tiles, 676 split 2 ways).  Not where the
+    // 64×64 or 96×64 tiles below run at once, more of them than these (166×2752×4224, 44 of these: 26.9 µs, 20.0 as
+    // 64×64 ones; 670×1664×4224 28.5 and, as 96×64 ones, 23.4; 300×4288×4224, 268 of those, 30.2 and 29.6).
     p = {96, 128, 1, 4, 3, 1, 0, 2};
   else if (t64 <= cus) {
-    // Split only while every split keeps at least 32 k steps: shorter ones spend more on the pipeline's
-    // fill, the partial sums and their finish than the extra workgroups win (750 frames of GigaAM, whose
-    // 768 × 3072 projections split in two and finished with the norm: 2 567 µs per call, whole 2 423).
-    while (p.split < 4 && t64 * p.split < 2L * cus && k % (2 * p.split * 64) == 0 && k / (2 * p.split * 64) >= 32)
-      p.split *= 2;
-    // Unsplit: two k groups of 4 wavefronts over a 4-slot ring (one workgroup per CU; the 750-frame
+    // Two k groups of 4 wavefronts over a 4-slot ring (one workgroup per CU; the 750-frame
     // 1024 × 1024 projections 9.5 against 10.0 µs in the step; deeper rings alone are slower there:
-    // 10.8 for 5 slots, 11.4 for 8).
-    if (p.split == 1 && k % 128 == 0) p = {64, 64, 2, 2, 4, 1, 0, 2};
+    // 10.8 for 5 slots, 11.4 for 8).  No split of k here: its partial sums and their finish cost more than the
+    // extra workgroups win (409×1856×4992 24.5 in two splits, 21.1 whole; 549×1664×4736 F16 23.8 and 19.1; 750
+    // frames of GigaAM, whose 768 × 3072 projections split in two and finished with the norm: 2 567 µs per call,
+    // whole 2 423).
+    if (k % 128 == 0) p = {64, 64, 2, 2, 4, 1, 0, 2};
   } else if (t64 < 2L * cus && !(f16 && (k % 128 || (t9664 > cus && k <= 1024))))
     // One to two 64×64 tiles per CU (the 750-frame pointwise projection, 750 × 2048 × 1024): 96×64
     // tiles of one row of 2 wavefronts in two k groups, one workgroup per CU (11.7 against 12.7 µs
