@@ -55,13 +55,14 @@ def test_k_wavefronts_need_k_to_split(gpu, m, n, k, wtype, plan):
     check(gpu, m, n, k, wtype, plan)
 
 
-# One to two 64x64 tiles per CU: 96x64 tiles in two k groups while those run at once and k has pairs of steps,
-# else 64x64 tiles, for quantized weights and few rows by k wavefronts.
+# One to two 64x64 tiles per CU: 96x64 tiles in two k groups where k has pairs of steps, else 64x64 tiles; few rows
+# whose 96x64 tiles do not run at once by k wavefronts with quantized weights, on 64x64 tiles with F16 ones.
 @pytest.mark.parametrize("m,n,k,wtype,plan", [
     (750, 2048, 1024, wa.Q8_0, "96x64_w1x2_n2_k2"), (750, 2048, 1024, wa.F16, "96x64_w1x2_n2_k2"),
     (765, 1408, 512, wa.F16, "96x64_w1x2_n2_k2"), (513, 2176, 896, wa.Q4_0, "96x64_w1x2_n2_k2"),
     (500, 3072, 1024, wa.Q8_0, KW64), (500, 3072, 1024, wa.F16, "64x64_w2x2_n3"), (623, 2688, 1536, wa.F16, "96x64_w1x2_n2_k2"),
-    (392, 3520, 1728, wa.Q4_0, KW64), (339, 3392, 1088, wa.Q8_0, KW64), (918, 1472, 1984, wa.F16, "64x64_w2x2_n3")])
+    (392, 3520, 1728, wa.Q4_0, KW64), (339, 3392, 1088, wa.Q8_0, KW64), (918, 1472, 1984, wa.F16, "64x64_w2x2_n3"),
+    (1393, 1344, 2880, wa.Q4_0, "64x64_w2x2_n3"), (1286, 1024, 2496, wa.Q8_0, "64x64_w2x2_n3")])
 @pytest.mark.parametrize("out16", [False, True])
 def test_one_to_two_tiles_per_cu(gpu, m, n, k, wtype, plan, out16):
     check(gpu, m, n, k, wtype, plan, out16)

@@ -119,12 +119,13 @@ GemmPlan gemm_plan_for(const wh_ctx *ctx, int m, int cols, int k, int type) {
     // frames of GigaAM, whose 768 × 3072 projections split in two and finished with the norm: 2 567 µs per call,
     // whole 2 423).
     if (k % 128 == 0) p = {64, 64, 2, 2, 4, 1, 0, 2};
-  } else if (t64 < 2L * cus && !(f16 && (k % 128 || (t9664 > cus && k <= 1024))))
+  } else if (t64 < 2L * cus && k % 128 == 0 && !(f16 && t9664 > cus && k <= 1024))
     // One to two 64×64 tiles per CU (the 750-frame pointwise projection, 750 × 2048 × 1024): 96×64
     // tiles of one row of 2 wavefronts in two k groups, one workgroup per CU (11.7 against 12.7 µs
-    // in the step for 64×64 tiles; 12.2 with 4 slots).  F16 weights stay on 64×64 tiles over an odd number of
-    // steps (918×1472×1984 15.7 against 20.4) and over more than a 96×64 tile per CU of a short k
-    // (937×1728×1024 11.6 against 12.9; 623×2688×1536 15.4 and 16.0, 571×3520×1920 20.7 and 19.5).
+    // in the step for 64×64 tiles; 12.2 with 4 slots).  64×64 tiles stay where there are no two groups, an odd
+    // number of steps (1393×1344×2880 Q4_0 24.2 against 34.0, 918×1472×1984 F16 15.7 against 20.4), and with F16
+    // weights over more than a 96×64 tile per CU of a short k (937×1728×1024 11.6 against 12.9; 623×2688×1536 15.4
+    // and 16.0, 571×3520×1920 20.7 and 19.5).
     p = {96, 64, 1, 2, 2, 1, 0, 2};
   // Few tiles: wavefronts that split k (gemm_kw_kernel), the smallest of its tiles that still run at once
   // (one workgroup per CU), whose chain of steps is then the shortest.  µs per encoder call with that one
