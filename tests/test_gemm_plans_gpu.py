@@ -78,3 +78,31 @@ def test_one_to_two_tiles_per_cu(gpu, m, n, k, wtype, plan, out16):
     (757, 1792, 4096, wa.F16, "128x128_w2x2_n2_s4")])
 def test_long_k(gpu, m, n, k, wtype, plan):
     check(gpu, m, n, k, wtype, plan)
+
+
+# About a tile per CU and more: each tile of the choice by rounds, for quantized and F16 weights, over rows and columns
+# that end inside a tile, a k without pairs of steps (960) and short ones (256); and where the choice begins.
+@pytest.mark.parametrize("m,n,k,wtype,plan", [
+    (2970, 900, 256, wa.Q8_0, "96x128_w1x4_n3_k2"),
+    (2970, 900, 256, wa.F16, "96x128_w1x4_n3_k2"),
+    (3220, 516, 960, wa.Q8_0, "96x128_w1x4_n3"),
+    (3220, 516, 960, wa.F16, "96x128_w1x4_n3"),
+    (3503, 772, 256, wa.Q4_0, "128x128_w2x4_n3"),
+    (3503, 772, 256, wa.F16, "128x128_w2x4_n3"),
+    (3680, 3204, 960, wa.Q8_0, "128x128_w2x2_n2"),
+    (2309, 2489, 256, wa.F16, "128x128_w2x2_n2"),
+    (3000, 4096, 1024, wa.Q8_0, "192x128_w2x4_n2"),
+    (2947, 1284, 256, wa.Q4_0, "192x128_w2x4_n2"),
+    (2947, 1284, 256, wa.F16, "192x128_w2x4_n2"),
+    (2502, 2336, 2048, wa.Q8_0, "256x128_w2x4_n3"),
+    (2502, 2336, 2048, wa.F16, "256x128_w2x4_n3"),
+    (22384, 288, 1984, wa.F16, "192x256_w2x4_n2"),
+    (3894, 3097, 768, wa.Q4_0, "256x256_w2x4_n2"),
+    (9477, 1280, 5120, wa.Q8_0, "192x256_w2x4_n2"),
+    (3894, 3097, 768, wa.F16, "256x256_w2x4_n2"),
+    (750, 4096, 1024, wa.Q8_0, "96x128_w1x4_n3_k2"),
+    (30020, 256, 256, wa.Q8_0, "128x128_w2x4_n3"),
+    (4633, 480, 512, wa.Q8_0, "96x128_w1x4_n3_k2"),
+    (5163, 512, 192, wa.Q4_0, "64x64_w2x2_n3"), (5735, 512, 192, wa.F16, "64x64_w2x2_n3")])
+def test_choice_by_rounds(gpu, m, n, k, wtype, plan):
+    check(gpu, m, n, k, wtype, plan)

@@ -155,28 +155,6 @@ def test_gemm_round_tiles(gpu, wtype, plan):
     test_gemm_every_plan(gpu, wtype, plan)
 
 
-# The choice by rounds, at shapes that take each of its tiles, the last ones partly filled, a k without
-# whole pairs of steps and cols past the last tile: against one tile shape that walks the same k order.
-@pytest.mark.parametrize("m,n,k", [(1031, 2048, 1024), (2011, 3072, 768), (1100, 3072, 768), (3600, 1024, 1024),
-                                   (1500, 4160, 1024), (1500, 4100, 960), (2000, 4096, 1024), (3600, 4096, 1024),
-                                   (2900, 4160, 320)])
-def test_gemm_choice_by_rounds(gpu, m, n, k):
-    w = np.random.default_rng(k).normal(0, 0.02, (n, k)).astype(np.float32)
-    l = gpu.linear([(ox.quantize(w, wa.Q8_0), wa.Q8_0, k, n)], rnd(n, 2))
-    ah = gpu.upload(rnd(m * k, 3).reshape(m, k).astype(np.float16))
-    got = []
-    for plan in ("", "128,128,2,4,3,1"):
-        gpu.tune("gemm_plan", plan)
-        try:
-            cb = gpu.buffer(m * l.width)
-            gpu.gemm_h(ah, l, cb, m, wa.BIAS)
-            got.append(gpu.read(cb, (m, l.width)))
-        finally:
-            gpu.tune("gemm_plan", "")
-    # The same products in f32 in one or two runs of k steps: sums in another order, as above.
-    close(got[0], got[1], tol=2e-5 * max(1.0, float(np.abs(got[1]).max())), what=f"{m}x{n}x{k}")
-
-
 # The k-wavefront kernel's tiles (pipeline 3), over rows and columns that end inside a tile, k steps that
 # leave wavefronts with none (64, 320) or unequal shares (960), a row count that needs padding columns
 # (257 -> 320) and dual columns.

@@ -37,27 +37,28 @@
 
 // Shapes of about one 128×128 tile per CU or more: whole k, and the tile shape whose rounds over the CUs take
 // the least time.  Such a GEMM is bound by its last, partly filled round as much as by the tiles' own rate, so
-// no single tile is best over a range of rows (µs, Q8_0): 3000×4096×1024 is 51.0 as 96×128 tiles in two k
-// groups (3 rounds and an eighth of one) and 34.5 as 192×128 ones (one round, two workgroups per CU);
-// 3600×4096×1024 61.0 and, as 256×256 ones, 40.3; 2500×3840×1280 53.6 -> 37.0; 11616×1280×5120 198.6 -> 166.6.
-// Over 82 shapes of 1100 .. 11616 rows, 768 .. 5120 columns and k of 768 .. 5120 the choice below is within 1%
-// of the best of these tiles in the mean and 1.15 times as fast as one tile per range of tile counts.
+// no single tile is best over a range of rows (µs, Q8_0): 3600×4096×1024 is 61.0 as 96×128 tiles in two k
+// groups (4 rounds and three quarters of one) and 40.3 as 256×256 ones; 3000×4096×1024 51.0 (4 rounds) and 34.5 as
+// 192×128 ones (one round, two workgroups per CU); 2500×3840×1280 53.6 -> 37.0; 11616×1280×5120 198.6 -> 166.6.
+// Over 312 random shapes of 600 to 60000 rows, 256 to 5120 columns and k of 64 to 5120 in the three weight types
+// the choice below is within 3% of the best of these tiles in the mean, 1.18 times as fast as one tile per range
+// of tile counts.  Below k = 1024 a round costs what its launch, its ring's fill and its stores cost, much the
+// same for one or two workgroups per CU and most for 256×256 tiles: from the line above 1024 carried down, those
+// seemed the cheapest for a short k (10236×2432×384 43.4 as 256×256 ones, 31.7 as 128×128 ones).
 struct TileRounds {
   GemmPlan plan;
-  int per_cu, per_cu_f16;  // workgroups that share a CU (LDS), with quantized and with F16 weights; 0: not taken
-  float t[3][2];  // a round with 1 .. per_cu workgroups per CU: t[·][0] + t[·][1] · k / 1024 µs, measured at k of 1024 .. 5120
+  int per_cu, per_cu_f16;  // workgroups that share a CU (LDS), with quantized and with F16 weights
+  float t[3][3];  // a round with 1 .. per_cu workgroups per CU, µs: as k goes to 0, at k = 1024, per 1024 of k from there
 };
 constexpr TileRounds TILE_ROUNDS[] = {
-    {{96, 128, 1, 4, 3, 1, 0, 2}, 1, 1, {{7.0f, 6.5f}}},
-    {{96, 128, 1, 4, 3, 1}, 2, 1, {{6.0f, 8.0f}, {8.3f, 13.2f}}},
-    {{128, 128, 2, 4, 3, 1}, 2, 1, {{7.0f, 8.2f}, {7.5f, 18.2f}}},
-    {{128, 128, 2, 2, 2, 1}, 3, 2, {{7.8f, 9.0f}, {8.0f, 17.7f}, {8.7f, 26.8f}}},
-    {{192, 128, 2, 4, 2, 1}, 2, 2, {{8.5f, 11.5f}, {4.0f, 27.5f}}},
-    // (F16 weights have no dequantization that wavefronts of fewer columns would repeat)
-    {{256, 128, 2, 4, 3, 1}, 1, 0, {{9.2f, 16.6f}}},
-    {{256, 128, 4, 2, 2, 1}, 0, 1, {{9.2f, 16.6f}}},
-    {{192, 256, 2, 4, 2, 1}, 1, 1, {{6.7f, 25.8f}}},
-    {{256, 256, 2, 4, 2, 1}, 1, 1, {{8.4f, 31.6f}}},
+    {{96, 128, 1, 4, 3, 1, 0, 2}, 1, 1, {{7.0f, 13.5f, 6.5f}}},
+    {{96, 128, 1, 4, 3, 1}, 2, 1, {{9.0f, 14.0f, 8.0f}, {16.0f, 21.5f, 13.2f}}},
+    {{128, 128, 2, 4, 3, 1}, 2, 1, {{7.0f, 15.2f, 8.2f}, {7.3f, 25.7f, 18.2f}}},
+    {{128, 128, 2, 2, 2, 1}, 3, 2, {{7.5f, 16.8f, 9.0f}, {7.7f, 25.7f, 17.7f}, {16.5f, 35.5f, 26.8f}}},
+    {{192, 128, 2, 4, 2, 1}, 2, 2, {{7.0f, 20.0f, 11.5f}, {8.5f, 31.5f, 27.5f}}},
+    {{256, 128, 2, 4, 3, 1}, 1, 1, {{10.0f, 25.8f, 16.6f}}},
+    {{192, 256, 2, 4, 2, 1}, 1, 1, {{8.5f, 32.5f, 25.8f}}},
+    {{256, 256, 2, 4, 2, 1}, 1, 1, {{26.0f, 40.0f, 31.6f}}},
 };
 
 GemmPlan least_rounds(int cus, int m, int cols, int k, bool f16) {
@@ -66,9 +67,12 @@ GemmPlan least_rounds(int cus, int m, int cols, int k, bool f16) {
   for (const TileRounds &r : TILE_ROUNDS) {
     const GemmPlan &p = r.plan;
     const int per_cu = f16 ? r.per_cu_f16 : r.per_cu;
-    if (!per_cu || k % (64 * p.wk)) continue;
+    if (k % (64 * p.wk)) continue;
     const long tiles = (long)((cols + p.bn - 1) / p.bn) * ((m + p.bm - 1) / p.bm), slots = (long)cus * per_cu;
-    auto round = [&](long wgs) { return r.t[(wgs - 1) / cus][0] + r.t[(wgs - 1) / cus][1] * (float)k / 1024.0f; };
+    auto round = [&](long wgs) {
+      const float *c = r.t[(wgs - 1) / cus], x = (float)k / 1024.0f;
+      return x < 1.0f ? c[0] + (c[1] - c[0]) * x : c[1] + c[2] * (x - 1.0f);
+    };
     const float t = (float)(tiles / slots) * round(slots) + (tiles % slots ? round(tiles % slots) : 0.0f);
     if (least == 0.0f || t < least) least = t, best = p;
   }
@@ -85,10 +89,11 @@ GemmPlan gemm_plan_for(const wh_ctx *ctx, int m, int cols, int k, int type) {
   const long t128 = (long)((cols + 127) / 128) * ((m + 127) / 128), t64 = (long)((cols + 63) / 64) * ((m + 63) / 64);
   const long t9664 = (long)((cols + 63) / 64) * ((m + 95) / 96);
   GemmPlan p{64, 64, 2, 2, 3, 1};
-  if (t128 * 4 >= 3L * cus || (t128 * 2 > cus && m >= 1024))
+  if (t128 * 4 >= 3L * cus || (t128 * 2 > cus && m >= 1024 && k >= 512))
     // Three quarters of a 128×128 tile per CU or more (the FFN's first projection at 750 frames: 96×128 tiles
     // in two k groups, 256 of them), of many rows half a tile (1100×2048×1024 14.9 -> 12.0 µs, 2500×1024×1024
-    // 15.7 -> 13.8 as 96×128 tiles); with fewer rows 64×64 tiles stay ahead (the 750-frame qkv projection, 144
+    // 15.7 -> 13.8 as 96×128 tiles), over a long enough k (4633×480×512 10.1 -> 8.5, but 5163×512×192 7.3 on 64×64
+    // tiles, 8.0 on those); with fewer rows 64×64 tiles stay ahead (the 750-frame qkv projection, 144
     // of 128×128: the 60 s step 4.32 ms, 4.51 as 96×128 ones).
     p = least_rounds(cus, m, cols, k, f16);
   else if (t128 * 4 <= cus && k % (4 * 64) == 0 && k / (4 * 64) >= 16)

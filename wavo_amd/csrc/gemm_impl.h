@@ -1379,7 +1379,7 @@ int launch_lds_t(wh_ctx *ctx, const _Float16 *a, const wh_linear *l, void *c, in
     PLAN(64, 64, 2, 2, 3)
     PLAN(128, 128, 2, 4, 2)  // tuning only: 2 to 4% behind the tiles that the choice takes
     PLAN(128, 128, 2, 2, 2)
-    PLAN(256, 128, 4, 2, 2)
+    PLAN(256, 128, 4, 2, 2)  // tuning only: as fast as the three slots below, or 1.2 times their time
     PLAN(256, 128, 2, 4, 3)
     PLAN(192, 128, 2, 4, 2)
     PLAN(192, 256, 2, 4, 2)
