@@ -103,6 +103,8 @@ def test_long_k(gpu, m, n, k, wtype, plan):
     (750, 4096, 1024, wa.Q8_0, "96x128_w1x4_n3_k2"),
     (30020, 256, 256, wa.Q8_0, "128x128_w2x4_n3"),
     (4633, 480, 512, wa.Q8_0, "96x128_w1x4_n3_k2"),
-    (5163, 512, 192, wa.Q4_0, "64x64_w2x2_n3"), (5735, 512, 192, wa.F16, "64x64_w2x2_n3")])
+    (5163, 512, 192, wa.Q4_0, "64x64_w2x2_n3"), (5735, 512, 192, wa.F16, "64x64_w2x2_n3"),
+    (500, 4096, 512, wa.F16, "96x128_w1x4_n3_k2"), (491, 4544, 256, wa.F16, "96x128_w1x4_n3_k2"),
+    (500, 4096, 512, wa.Q8_0, KW64)])
 def test_choice_by_rounds(gpu, m, n, k, wtype, plan):
     check(gpu, m, n, k, wtype, plan)

@@ -89,12 +89,13 @@ GemmPlan gemm_plan_for(const wh_ctx *ctx, int m, int cols, int k, int type) {
   const long t128 = (long)((cols + 127) / 128) * ((m + 127) / 128), t64 = (long)((cols + 63) / 64) * ((m + 63) / 64);
   const long t9664 = (long)((cols + 63) / 64) * ((m + 95) / 96);
   GemmPlan p{64, 64, 2, 2, 3, 1};
-  if (t128 * 4 >= 3L * cus || (t128 * 2 > cus && m >= 1024 && k >= 512))
+  if (t128 * 4 >= 3L * cus || (m >= 1024 && t128 * 2 > cus && k >= 512) || (f16 && t64 >= 2L * cus && k >= 256))
     // Three quarters of a 128×128 tile per CU or more (the FFN's first projection at 750 frames: 96×128 tiles
     // in two k groups, 256 of them), of many rows half a tile (1100×2048×1024 14.9 -> 12.0 µs, 2500×1024×1024
     // 15.7 -> 13.8 as 96×128 tiles), over a long enough k (4633×480×512 10.1 -> 8.5, but 5163×512×192 7.3 on 64×64
-    // tiles, 8.0 on those); with fewer rows 64×64 tiles stay ahead (the 750-frame qkv projection, 144
-    // of 128×128: the 60 s step 4.32 ms, 4.51 as 96×128 ones).
+    // tiles, 8.0 on those); with fewer rows 64×64 tiles stay ahead (the 750-frame qkv projection, 144 of 128×128:
+    // the 60 s step 4.32 ms, 4.51 as 96×128 ones), up to two per CU with F16 weights, whose tiles they then fetch
+    // in step from a part of the memory's channels (500×4096×512 10.5 -> 8.4, 491×4544×256 9.6 -> 6.9).
     p = least_rounds(cus, m, cols, k, f16);
   else if (t128 * 4 <= cus && k % (4 * 64) == 0 && k / (4 * 64) >= 16)
     // Long k over few tiles (the FFN's down projection, 750 × 1024 × 4096): k split 4 ways over
