@@ -87,7 +87,7 @@ void *wh_stream(wh_ctx *ctx);
  * per device tier, src/gpu/mod.rs:50-107).  Only an explicit call changes them; a fresh context
  * chooses every launch plan itself.  Keys:
  *   "gemm_plan"        "bm,bn,wm,wn,slots,split[,pipeline[,kgroups]]" for every GEMM of the main kernel
- *                      ("" clears);
+ *                      ("" clears; kgroups 1 or 2, the wavefronts of a workgroup for pipeline 3);
  *   "gemm_shape_plans" "m,cols,k:bm,bn,wm,wn,slots,split[,pipeline[,kgroups]];..." per call shape ("" clears);
  *   "gemm_kernel_only" "1": a k-split GEMM call stops after its GEMM kernel and leaves c unwritten
  *                      (to time that kernel alone, as a model step runs it); "0" restores;

@@ -80,3 +80,26 @@ def test_whisper_window_past_the_model(gpu):
     m.whisper_begin(enc, frames)
     m.free()
     still_works(gpu)
+
+
+def test_plans_out_of_range_are_refused(gpu):
+    """k groups past 2 belong to the k-wavefront kernel (pipeline 3) alone, and that kernel, forced by a plan, refuses
+    rows past its 32-bit offsets instead of wrapping them; the context keeps working."""
+    for key, head in (("gemm_plan", ""), ("gemm_shape_plans", "40,64,256:")):
+        for bad in ("64,64,2,2,3,1,0,3", "64,64,2,2,3,1,0,16", "32,32,1,1,2,1,3,9"):
+            with pytest.raises(wa.WavoError) as e:
+                gpu.tune(key, head + bad)
+            assert e.value.code == wa.EARG, (key, bad)
+    m, n, k = 1 << 21, 32, 1024  # 4 GiB of f16 rows
+    raw = gguf.encode(np.zeros(n * k, np.float32), gguf.Q8_0)
+    l = gpu.linear([(raw, wa.Q8_0, k, n)], np.ones(n, np.float32))
+    a, c = gpu.buffer(m * k // 2), gpu.buffer(m * n)
+    gpu.tune("gemm_plan", "32,32,1,1,2,1,3,8")
+    try:
+        with pytest.raises(wa.WavoError) as e:
+            gpu.gemm_h(a, l, c, m, wa.BIAS)
+        assert e.value.code == wa.EARG and "4 GiB" in str(e.value)
+        gpu.gemm_h(gpu.upload(np.zeros((40, k), np.float16)), l, c, 40, wa.BIAS)
+        assert np.array_equal(gpu.read(c, (40, n)), np.ones((40, n), np.float32))
+    finally:
+        gpu.tune("gemm_plan", "")

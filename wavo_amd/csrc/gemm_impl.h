@@ -1302,26 +1302,28 @@ int lds_launch(wh_ctx *ctx, dim3 grid, const LdsArgs &a, bool split, bool out16)
   }
 }
 
-// The k-wavefront kernel of plan p (*ok: built).
+// The k-wavefront kernel of plan p; false: not built.
 template <int WT>
-int kw_launch(wh_ctx *ctx, dim3 grid, const LdsArgs &a, const GemmPlan &p, bool out16, bool *ok) {
+bool kw_launch(wh_ctx *ctx, dim3 grid, const LdsArgs &a, const GemmPlan &p, bool out16) {
 #define KW(TM, TN, WK)                                                                              \
   if (p.bm == 32 * TM && p.bn == 32 * TN && p.wk == WK && p.split == 1) {                           \
     if (out16) wh_launch(ctx, gemm_kw_kernel<WT, TM, TN, WK, true>, grid, 64 * WK, 0, a);           \
     else wh_launch(ctx, gemm_kw_kernel<WT, TM, TN, WK, false>, grid, 64 * WK, 0, a);                \
-    *ok = true;                                                                                     \
+    return true;                                                                                    \
   }
   KW(1, 1, 8)
   KW(1, 2, 8)
-  KW(2, 2, 4)
+  KW(2, 2, 4)  // (F16 weights: tuning only)
 #undef KW
-  return WH_OK;
+  return false;
 }
 
 template <int WT>
 int launch_lds_t(wh_ctx *ctx, const _Float16 *a, const wh_linear *l, void *c, int m, int ldc, int epi, float alpha,
                  bool out16, float *part, int *splits, const HeadsOut *ho, int nho) {
   GemmPlan p = gemm_plan_for(ctx, m, l->cols, l->k, l->type);
+  if (p.pipe == PIPE_KW && (size_t)m * l->k >= ((size_t)1 << 31))  // (a forced plan)
+    return wh_fail(ctx, WH_EARG, "gemm: the k-wavefront kernel reaches 4 GiB of a, not %d rows of %d", m, l->k);
   if ((p.split > 1 && !part) || nho) p.split = 1;  // packed ranges are written by the tiles' own epilogue
   for (int i = 0; i < nho; i++)  // packed ranges of whole 64-column tiles only
     if (ho[i].col0 % p.bn || ho[i].cols % p.bn) p = {64, 64, 2, 2, 3, 1};
@@ -1365,9 +1367,7 @@ int launch_lds_t(wh_ctx *ctx, const _Float16 *a, const wh_linear *l, void *c, in
     ProfScope prof(ctx, name, args.skip ? 0.0 : 2.0 * m * l->rows * l->k, args.skip ? 0.0 : bytes);
     const bool sp = p.split > 1;
     bool ok = false;
-    if (p.pipe == PIPE_KW) {
-        if (int rc = kw_launch<WT>(ctx, grid, args, p, out16, &ok)) return rc;
-    }
+    if (p.pipe == PIPE_KW) ok = kw_launch<WT>(ctx, grid, args, p, out16);
 #define PLANK(BM, BN, WM, WN, NS, PIPE, WK)                                                                       \
   if (!ok && p.bm == BM && p.bn == BN && p.wm == WM && p.wn == WN && p.ns == NS && p.pipe == PIPE && p.wk == WK) { \
     if (int rc = lds_launch<WT, BM, BN, WM, WN, NS, PIPE, WK>(ctx, grid, args, sp, out16)) return rc;               \

@@ -376,9 +376,9 @@ int wh_tune(wh_ctx *ctx, const char *key, const char *value) {
   if (!strcmp(key, "gemm_plan")) {
     int o[8] = {0, 0, 0, 0, 0, 0, 0, 0};
     if (*v && (sscanf(v, "%d,%d,%d,%d,%d,%d,%d,%d", &o[0], &o[1], &o[2], &o[3], &o[4], &o[5], &o[6], &o[7]) < 6 ||
-               o[5] < 1 || o[5] > 4 || o[7] < 0 || o[7] > 16))
+               o[5] < 1 || o[5] > 4 || o[7] < 0 || o[7] > (o[6] == 3 ? 8 : 2)))
       return wh_fail(ctx, WH_EARG,
-                     "wh_tune gemm_plan: \"bm,bn,wm,wn,stages,split[,pipeline[,kgroups]]\" (split 1..4, kgroups 1..16) or \"\"");
+                     "wh_tune gemm_plan: \"bm,bn,wm,wn,stages,split[,pipeline[,kgroups]]\" (split 1..4, kgroups 1..2, wavefronts 1..8 of pipeline 3) or \"\"");
     memcpy(ctx->gemm_plan, o, sizeof o);
   } else if (!strcmp(key, "gemm_shape_plans")) {
     ctx->gemm_shape_plans.clear();
@@ -386,7 +386,7 @@ int wh_tune(wh_ctx *ctx, const char *key, const char *value) {
       std::array<int, 11> o{};
       if (sscanf(q, "%d,%d,%d:%d,%d,%d,%d,%d,%d,%d,%d", &o[0], &o[1], &o[2], &o[3], &o[4], &o[5], &o[6], &o[7], &o[8],
                  &o[9], &o[10]) < 9 ||
-          o[8] < 1 || o[8] > 4 || o[10] < 0 || o[10] > 16)
+          o[8] < 1 || o[8] > 4 || o[10] < 0 || o[10] > (o[9] == 3 ? 8 : 2))
         return wh_fail(ctx, WH_EARG,
                        "wh_tune gemm_shape_plans: \"m,cols,k:bm,bn,wm,wn,stages,split[,pipeline[,kgroups]];...\"");
       ctx->gemm_shape_plans.push_back(o);
