@@ -110,6 +110,26 @@ def test_parakeet_attention_reads_in_place(gpu, small, seconds):
             assert np.array_equal(direct, got), (key, float(np.abs(direct - got).max()))
 
 
+def test_parakeet_packed_ranges_off_the_chosen_tile(gpu, tmp_path):
+    """A width (576) whose q, K and V ranges start inside the 128-column tiles that the projection of 1200 frames
+    would take: it takes 64-column ones, whole tiles of which the packed ranges are."""
+    config = dict(synth.SMALL["parakeet"], layers=1, d=576, heads=9, d_ff=1152)
+    path = synth.write_model(str(tmp_path / "m.gguf"), config, 0, gguf.Q8_0)
+    mel = synth.parakeet_mel(synth.audio(96.0, 11))
+    m, om = wa.Model(gpu, path), ox.Model(path)
+    t = m.frames(mel.shape[0])[0]
+    gpu.profile(1)
+    try:
+        got = m.encode(mel)
+        names = [x["kernel"] for x in gpu.profile_read()]
+    finally:
+        gpu.profile(0)
+    assert any(x.startswith(f"gemm_q8_0_64x64_w2x2_n3 {t}x1728x576") for x in names), names
+    assert not any("pack" in x for x in names), names
+    want = om.encode(mel)
+    assert got.shape == want.shape and rel_l2(got, want) < ENCODER_TOL, rel_l2(got, want)
+
+
 def test_parakeet_kestrel_valid(gpu):
     # The kestrel length masking: the last mel frame is padding (src/parakeet/mod.rs:140-141).
     path = synth.model_path("parakeet", small=True, directory=MODELS)

@@ -237,6 +237,12 @@ def test_gemm_tile_orders_agree(gpu, plan):
         close(outs[0], want, tol=2e-5 * max(1.0, float(np.abs(want).max())), what=f"plan {plan}, n {n}")
 
 
+# The same for the k-wavefront kernel, which renumbers its tiles itself, and the tiles of 192 rows.
+@pytest.mark.parametrize("plan", ["32,32,1,1,2,1,3,8", "32,64,1,1,2,1,3,8", "64,64,1,1,2,1,3,4", "192,128,2,4,2,1", "192,256,2,4,2,1"])
+def test_gemm_tile_orders_agree_few_rows_and_many(gpu, plan):
+    test_gemm_tile_orders_agree(gpu, plan)
+
+
 def test_gemm_rejects_internal_epilogues(gpu):
     # The library's own epilogues past WH_TANH (the conv module's GLU) are not callers' to ask for.
     m, n, k = 4, 64, 64
