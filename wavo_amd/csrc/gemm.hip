@@ -1,9 +1,9 @@
 // The quantized GEMM of Pass::gemm (src/gpu/mod.rs:1394-1426) on gfx950 matrix cores:
 //   c[m][j] = epi(Σ_k h(a[m][k]) · h(W[j][k]) + bias[j]),  h = round to f16 (RNE), f32 accumulate,
-// as gemm.wgsl:170-242 and the CPU backend (src/cpu/gemm.rs:126-177) define it.  W stays in HBM as
-// the GGUF stores it (src/gguf.rs:14-38; the GEMVs read it so): Q8_0 34-byte blocks (f16 scale + 32 int8),
-// Q4_0 18-byte blocks (f16 scale + 16 bytes of nibbles), F16 or F32 rows; and once more in tiles of 32 rows
-// × 64 k in the order the matrix-core lanes load them (WTile, weight_tiles_kernel), for the kernels here.
+// as gemm.wgsl:170-242 and the CPU backend (src/cpu/gemm.rs:126-177) define it.  The GGUF's rows
+// (src/gguf.rs:14-38; Q8_0 34-byte blocks (f16 scale + 32 int8), Q4_0 18-byte blocks (f16 scale + 16 bytes of
+// nibbles), F16 or F32) are laid out, for the matrix-core kernels here, in tiles of 32 rows × 64 k in the order
+// their lanes load them (WTile, weight_tiles_kernel), once, when the layer is created.
 //
 // Main kernel (gemm_lds_kernel; k % 64 == 0, W in Q8_0 / Q4_0 / F16, `a` in f16): a ring of LDS stages
 // fed by the LDS DMA of gfx950 — per 64- or 128-wide k step, the a tile and W's tiles, all in 16-byte
@@ -18,14 +18,14 @@
 // bits, so f32 and the f16 multiply round the same value).  The epilogues of Epilogue::params
 // (src/gpu/mod.rs:445-455; gemm.wgsl:72-94) and the dual outputs are fused into the store, in f32
 // or, for a consumer that rounds its input to f16 anyway (another GEMM), in f16.  Shapes with too
-// few output tiles for the 256 CUs split k 2 or 4 ways into f32 partial sums that a second kernel
+// few output tiles for the 256 CUs and a long k split it 4 ways into f32 partial sums that a second kernel
 // adds in a fixed order before the epilogue.
 //
-// Few tiles (gemm_kw_kernel): the wavefronts of a workgroup split k and read W from tiles laid out for
-// their loads when the weights are created (weight_tiles_kernel).
+// Few tiles (gemm_kw_kernel): the wavefronts of a workgroup split k and read W's tiles straight into
+// registers.
 //
-// Fallback kernel (gemm_reg_kernel; any k % 32 == 0 and F32 weights): a double-buffered a tile in
-// LDS and W blocks loaded straight into registers.
+// Fallback kernel (gemm_reg_kernel; any k % 32 == 0, F32 weights and layers without tiles): a
+// double-buffered a tile in LDS and W's blocks as stored loaded straight into registers.
 #include <algorithm>
 #include <cstdio>
 #include <mutex>
@@ -81,8 +81,8 @@ GemmPlan least_rounds(int cus, int m, int cols, int k, bool f16) {
 
 // Chosen per GEMM shape from measurements on MI355X (random operands, inside the encoder step, or
 // replayed back to back for m ≥ 1024): many output tiles → the tile shape with the cheapest rounds; fewer
-// → 64×64 tiles of 4 wavefronts, and when even those leave CUs idle, k split 2 or 4 ways.  Ring slots
-// of 64-wide k steps (a slot is refilled NS steps ahead, so NS − 1 steps hide the DMA's latency).
+// → 96×128, 96×64 or 64×64 tiles in two k groups, wavefronts that split k, or, a long k over few tiles, k split
+// 4 ways.  Ring slots of 64-wide k steps (a slot is refilled NS steps ahead, so NS − 1 steps hide the DMA's latency).
 GemmPlan gemm_plan_for(const wh_ctx *ctx, int m, int cols, int k, int type) {
   const bool f16 = type == WH_F16;
   const int cus = ctx->cus > 0 ? ctx->cus : 256;
@@ -188,7 +188,7 @@ bool lds_path(const wh_linear *l, const void *c, int ldc) {
 }
 
 
-// The k-wavefront kernel's weight tiles from the GGUF bytes (see WTile): a lane of a tile per thread.
+// The weight tiles from the GGUF bytes (see WTile): a lane of a tile per thread.
 template <int WT>
 __global__ __launch_bounds__(256) void weight_tiles_kernel(const uint8_t *__restrict__ w, uint8_t *__restrict__ wt, int rows,
                                                            int nkt, size_t row_bytes, size_t lanes) {

@@ -267,19 +267,10 @@ __device__ __forceinline__ uint32_t lds_addr(const void *p) {
   return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void *)p;
 }
 
-// LDS DMA (counted by vmcnt): each lane copies 16 (dma16) or 4 (dma4) bytes at `src` to LDS byte
-// lds + 16·lane (4·lane); `lds` is wave-uniform.
-__device__ __forceinline__ void dma16(const void *src, uint32_t lds) {
-  asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src), "{m0}"(__builtin_amdgcn_readfirstlane(lds))
-               : "memory");
-}
-__device__ __forceinline__ void dma4(const void *src, uint32_t lds) {
-  asm volatile("s_nop 0\n\tglobal_load_lds_dword %0, off" ::"v"(src), "{m0}"(__builtin_amdgcn_readfirstlane(lds))
-               : "memory");
-}
 __device__ __forceinline__ void dma_wait() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
-// The same from a wave-uniform base address (SGPRs) plus a per-lane 32-bit byte offset, so that a
-// loop moves the whole DMA by scalar adds.  `lds` must be wave-uniform (it goes to M0).
+// LDS DMA (counted by vmcnt): each lane copies the 16 bytes at a wave-uniform base address (SGPRs) plus its
+// 32-bit byte offset, so that a loop moves the whole DMA by scalar adds, to LDS byte lds + 16·lane; `lds` must be
+// wave-uniform (it goes to M0).
 __device__ __forceinline__ void dma16s(const void *base, uint32_t off, uint32_t lds) {
   // (the base through readfirstlane: a scalar value even where the scalar registers run short; the
   // halves as unsigned 32-bit values, since readfirstlane returns int and must not sign-extend)
@@ -289,10 +280,6 @@ __device__ __forceinline__ void dma16s(const void *base, uint32_t off, uint32_t 
   const uint64_t bs = ((uint64_t)hi << 32) | (uint64_t)lo;
   asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(bs), "{m0}"(lds) : "memory");
 }
-__device__ __forceinline__ void dma4s(const void *base, uint32_t off, uint32_t lds) {
-  asm volatile("s_nop 0\n\tglobal_load_lds_dword %0, %1" ::"v"(off), "s"(base), "{m0}"(lds) : "memory");
-}
-
 // Two int8 of x (bytes 0-1, or 2-3 with HI) as two f16 (exact: |q| ≤ 128), by sub-dword operand
 // selection of the conversion itself (SDWA: sign-extended byte in, one half of the result out).
 template <bool HI>
@@ -309,8 +296,8 @@ __device__ __forceinline__ half2 i8_pair(uint32_t x) {
   return __builtin_bit_cast(half2, r);
 }
 
-// W as the k-wavefront kernel reads it (wh_linear::wt, made from the GGUF bytes when the weights are
-// created): tiles of 32 rows × 64 k, [row tile][k step], rows past the last one zeros.  A tile holds the
+// W as gemm_lds_kernel and gemm_kw_kernel read it (wh_linear::wt, made from the GGUF bytes when the weights
+// are created): tiles of 32 rows × 64 k, [row tile][k step], rows past the last one zeros.  A tile holds the
 // MFMA operand bytes of lane l = 32g + r (row r, k half g) in the order the lanes load them, 16 bytes per
 // lane and load, so a load is 1 KiB of consecutive bytes:
 //   Q8_0  load i: block i's elements 8g .. 8g + 7, then 16 + 8g .. 16 + 8g + 7 (substeps 2i and 2i + 1);
@@ -326,7 +313,8 @@ struct WTile {
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
-// The MFMA operand of substep S from a lane's loads of a tile: f16(q·d), as dequant_q8 / dequant_frag.
+// The MFMA operand of substep S from a lane's loads of a tile: f16(q·d), the exact conversion of q and one packed
+// f16 multiply by the block's scale (F16: the weights as they are).
 template <int WT, int S>
 __device__ __forceinline__ half8 tile_frag(const u32x4 (&q)[WTile<WT>::LOADS], uint32_t sc) {
   if constexpr (WT == WH_F16) {
@@ -717,7 +705,7 @@ __device__ __forceinline__ void store_c_tile(const LdsArgs &P, const float *cl, 
 // the current slot right after the barrier, and a stage has NS − 1 steps to land.  The loop is
 // unrolled by the ring length so that every LDS offset is an immediate.  The DMA of a stage is spread
 // over the wavefronts, each instruction issued once (an instruction costs the memory pipeline the same
-// ~16 cycles whatever its width, so W rows move in 16-byte chunks too).
+// ~16 cycles whatever its width, so all of them move 16 bytes a lane).
 //
 // LDS layout: the a stages (rows of 8 16-byte chunks, chunk c of row r at (c + r/2) % 8 — the 16
 // lanes that LDS serves together read 16 rows and hit all 64 banks once), then the W stages: the tiles'
@@ -742,7 +730,7 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void gemm_lds_kernel(LdsArgs P) 
   constexpr int WL = WTile<WT>::LOADS, WT1 = BN / 32;  // loads per tile, tiles per sub-stage
   constexpr bool WSC = WT != WH_F16;
   static_assert(WT1 <= 8, "the scales of a sub-stage in one load");
-  // A ring slot holds WK consecutive 64-wide k steps (sub-stages): the a tile's, then the W rows'.
+  // A ring slot holds WK consecutive 64-wide k steps (sub-stages): the a tile's, then W's tiles.
   constexpr int A_ST0 = BM * 128, W_SC0 = WT1 * WTile<WT>::DATA, W_ST0 = W_SC0 + (WSC ? 1024 : 0);
   constexpr int A_ST = WK * A_ST0, W_ST = WK * W_ST0, ST = A_ST + W_ST;
   constexpr int CROW = BN + 8;                                           // f32 per epilogue LDS row
@@ -754,7 +742,7 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void gemm_lds_kernel(LdsArgs P) 
   constexpr int NIA = A_ST / 1024;                              // a: 16-byte DMA instructions per stage
   constexpr int NIW = W_ST / 1024;                              // W: 16-byte DMA instructions per stage
   // The wavefronts that issue the DMA: all of them; in the ping-pong loop the a tile by all of them
-  // and the W rows by the four of the second group.
+  // and W's tiles by the four of the second group.
   constexpr int NWA = NWT, NWI = PIPE == 2 ? 4 : NWT;
   // Instructions per wavefront and stage: PA / PW at most; the first NIA % NWI (NIW % NWI) wavefronts
   // take one more than the others.  vmcnt immediates count PI = the fewest a wavefront issues per stage:
@@ -886,7 +874,7 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void gemm_lds_kernel(LdsArgs P) 
     // step; group 1 starts one barrier later.  Stage i is read by group 0 between barriers 2i + 1 and
     // 2i + 3 and by group 1 between 2i + 2 and 2i + 4, so its slot refills after barrier 2i + 4 with
     // stage i + NS: the a tile by all eight wavefronts during their MFMAs of step i + 1 (one DMA
-    // instruction after the first MFMA of each substep), the W rows by group 1 during its
+    // instruction after the first MFMA of each substep), W's tiles by group 1 during its
     // dequantization of step i + 1.  Stage i + 1 must land by barrier 2i + 3: group 0 waits for its part
     // at the end of its MFMAs of step i, group 1 at the end of its dequantization of step i.
     static_assert(WM == 2 && WN == 4 && NS >= 3, "two groups of four wavefronts, three or more slots");
@@ -908,7 +896,7 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void gemm_lds_kernel(LdsArgs P) 
             if (i == 0 && j == 0) dma16s(ab, aoff[SS], lds0 + slot_d * A_ST + alds[SS]);
         }
     };
-    // Prologue: stages 0 .. NS − 2, the a tiles by all, the W rows by group 1.
+    // Prologue: stages 0 .. NS − 2, the a tiles by all, W's tiles by group 1.
 #pragma unroll
     for (int s = 0; s < NS - 1; s++)
       if (s < nk) {
@@ -940,8 +928,8 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void gemm_lds_kernel(LdsArgs P) 
         for (int j = 0; j < TN; j++) asm volatile("" : "+v"(wf[s][j]));
       if (g1) {
         if (more) issue_w(kt + NS - 1, dslot);
-        // Group 1's a-tile part of stage kt + 1 (issued in its MFMAs of step kt − 1) and W rows of it
-        // have landed: only the W rows just issued may remain.
+        // Group 1's a-tile part of stage kt + 1 (issued in its MFMAs of step kt − 1) and W's tiles of it
+        // have landed: only the W tiles just issued may remain.
         if (kt + 1 < nk) {
           if (more) wait_vm<QW>();
           else dma_wait();
